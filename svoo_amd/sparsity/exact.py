@@ -6,7 +6,7 @@
 ``threshold`` of the row's mass.  The reference materialises fp32 probabilities, sorts every row
 and searches a cumulative sum; here the score matmul stays a library GEMM (bf16 scores, as the
 reference's ``torch.matmul`` of bf16 inputs) and ``svoo_exact_sparsity_counts`` finds each row's
-count with two histogram passes over the bf16 scores (no sort, no fp32 probability tensor).
+count from a histogram of the row's bf16 bit patterns (no sort, no fp32 probability tensor).
 
 Counting contract: weights ``e_j = float(exp(double(s_j - m)))`` with ``s_j = float(score_j) *
 scale`` in fp32 and ``m`` the row max; prefix masses in fp64 over the weights in descending order;

@@ -58,6 +58,40 @@ def test_counts_long_rows(gpu):
     assert np.array_equal(got, O.exact_sparsity_counts(sc, 0.0884, 0.95))
 
 
+@pytest.mark.parametrize("n,kind", [(8191, "normal"), (8193, "ties"), (32767, "heavy"), (32769, "normal"),
+                                    (65535, "equal"), (65536, "equal"), (65543, "peaked"), (100003, "equal")])
+def test_counts_at_the_row_length_rules(gpu, n, kind):
+    """Row lengths on both sides of the kernel's variants (vectors per thread, the segments of rows whose 16-bit counts
+    could overflow; a row of one value fills a single count), odd lengths, so that rows start off 16-byte addresses, and
+    a tensor that starts off one itself: the counts are the oracle's."""
+    from svoo_amd.sparsity import exact_counts_from_scores
+
+    say("exact counts at the length rules", n, kind)
+    sc = _scores(np.random.default_rng(n), 5, n, kind)
+    flat = torch.zeros(5 * n + 3, dtype=torch.bfloat16, device=gpu)
+    flat[3:] = torch.from_numpy(sc).to(torch.bfloat16).to(gpu).flatten()
+    for thr in (0.5, 0.95):
+        got = exact_counts_from_scores(flat[3:].view(5, n), 0.0884, thr).cpu().numpy()
+        assert np.array_equal(got, O.exact_sparsity_counts(sc, 0.0884, thr)), (n, kind, thr)
+
+
+def test_counts_of_masked_and_infinite_scores(gpu):
+    """-inf (masked) scores weigh nothing; a row with +inf or NaN has no finite mass and counts every score above its
+    lowest value, plus one."""
+    from svoo_amd.sparsity import exact_counts_from_scores
+
+    say("exact counts with -inf, +inf and NaN")
+    sc = _scores(np.random.default_rng(3), 4, 1001, "normal")
+    sc[0, 100:] = -np.inf
+    sc[2, 5] = np.inf
+    sc[3, 7] = np.nan
+    got = exact_counts_from_scores(torch.from_numpy(sc).to(torch.bfloat16).to(gpu), 0.0884, 0.9).cpu().numpy()
+    assert np.array_equal(got[:2], O.exact_sparsity_counts(sc[:2], 0.0884, 0.9))
+    for r in (2, 3):
+        low = int((sc[r] == np.nanmin(sc[r])).sum())
+        assert got[r] == 1001 - low + 1
+
+
 def test_compute_exact_attention_sparsity(gpu):
     from svoo_amd.sparsity import compute_exact_attention_sparsity
 
