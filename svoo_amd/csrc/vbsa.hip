@@ -25,7 +25,10 @@
 // the attention are not separate passes.
 // EAR variant (centroid compensation): the KV stream continues after the active tokens with the
 // (key, value) centroids of the inactive clusters, each scored q . kc_j / sqrt(D) + log(|K_j| + 1e-6),
-// so one online softmax covers both (the reference's token attention + log-sum-exp merge).
+// so one online softmax covers both (the reference's token attention + log-sum-exp merge).  The token part is padded
+// to whole tiles: half a tile of masked keys per item on average, for which every tile's copies use one scalar base
+// and 32-bit offsets.  That leaves registers for half and B-chunked items (12 heads x 32760 tokens, 100 x 500
+// clusters: 4.85 ms with full items only, 4.40 ms with all kinds).
 #include <mutex>
 #include <type_traits>
 
@@ -324,7 +327,7 @@ __device__ __forceinline__ int build_segments(const uint8_t* __restrict__ mrow, 
 }
 
 // EAR: compacts the inactive key clusters of one map row (ascending) with their score bias
-// log2(e) * log(|K_j| + 1e-6) into LDS.  Returns their count.
+// log2(e) * log(|K_j| + 1e-6) into LDS; the biases up to the next whole tile are -inf (no key).  Returns their count.
 __device__ __forceinline__ int build_centroids(const uint8_t* __restrict__ mrow, const int32_t* __restrict__ ksb,
                                                int kn, int32_t* cent_idx, float* cent_bias, long long* red) {
   const int tid = threadIdx.x, nt = blockDim.x;
@@ -341,8 +344,10 @@ __device__ __forceinline__ int build_centroids(const uint8_t* __restrict__ mrow,
       ++idx;
     }
   }
+  const int n = (int)tot;
+  if (tid < kKT && n + tid < (n + kKT - 1) / kKT * kKT) cent_bias[n + tid] = -INFINITY;
   __syncthreads();
-  return (int)tot;
+  return n;
 }
 
 // Segment containing stream position p (seg_cum ascending, seg_cum[0] == 0).
@@ -365,6 +370,15 @@ constexpr int kXcdRun = 8;
 __device__ __forceinline__ long long xcd_item(long long bid) {
   const long long x = bid % 8, j = bid / 8;
   return (j / kXcdRun) * (8 * kXcdRun) + x * kXcdRun + (j % kXcdRun);
+}
+
+// A wave-uniform pointer settled in scalar registers here (left to the compiler, the choice of an EAR copy's base
+// became a branch around every copy).
+__device__ __forceinline__ const uint16_t* uniform_ptr(const uint16_t* p) {
+  const unsigned long long u = (unsigned long long)(uintptr_t)p;
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
+  return (const uint16_t*)(uintptr_t)(((unsigned long long)hi << 32) | lo);
 }
 
 // ------------------------------------------------------------------------------------------ attention
@@ -435,7 +449,8 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
   __shared__ __attribute__((aligned(16))) uint16_t k1_s0[kS1], k1_s1[kS1], v1_s0[kS1], v1_s1[kS1];
   __shared__ long long red[kVWaves];
   __shared__ int32_t rowtab[HC ? 2 : 1][2][2][kKT];  // [stream][K/V][slot][tile position] -> token row
-  extern __shared__ int32_t seg_mem[];  // seg_start[kn], seg_cum[kn + 1] (EAR: cent_idx[kn], cent_bias[kn])
+  // EAR: cent_bias[kn rounded up to whole tiles], cent_idx[kn]; then seg_start[kn], seg_cum[kn + 1]
+  extern __shared__ __attribute__((aligned(16))) int32_t seg_mem[];
 
   const long long item = xcd_item(blockIdx.x);
   if (item >= total_items) return;
@@ -483,19 +498,15 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
     else
       return ob + (size_t)r * 128;
   };
-  // EAR: the centroid rows are addressed from the token base of the head, as rows at a signed offset
-  // (the host checks that the buffers are 256-byte congruent and that every row index fits int32), so
-  // the DMA path is the same as for token rows.
-  int crow_k = 0, crow_v = 0;
-  if constexpr (EAR) {
-    crow_k = (int)(((long long)(uintptr_t)(kc + (size_t)b * kn * 128) - (long long)(uintptr_t)kb) / 256);
-    crow_v = (int)(((long long)(uintptr_t)(vc + (size_t)b * kn * 128) - (long long)(uintptr_t)vb) / 256);
-  }
+  // EAR: the stream's token part is padded to whole tiles, so a tile's rows lie in one buffer: the tokens' up to
+  // tile ear_tile, the centroids' after it (a scalar choice of the copies' base)
+  const uint16_t* kcb = EAR ? kc + (size_t)b * kn * 128 : nullptr;
+  const uint16_t* vcb = EAR ? vc + (size_t)b * kn * 128 : nullptr;
 
-  int32_t* seg_start = seg_mem;
-  int32_t* seg_cum = seg_mem + kn;
-  int32_t* cent_idx = seg_cum + kn + 1;
-  float* cent_bias = (float*)(cent_idx + kn);
+  float* cent_bias = (float*)seg_mem;
+  int32_t* cent_idx = seg_mem + (kn + kKT - 1) / kKT * kKT;
+  int32_t* seg_start = EAR ? cent_idx + kn : seg_mem;
+  int32_t* seg_cum = seg_start + kn;
   int total = 0;
   const uint8_t* mrow = map + ((size_t)b * qn + ci) * kn;
   const int nseg_v = build_segments(mrow, koff + (size_t)b * (kn + 1), ks + (size_t)b * kn, kn, seg_start, seg_cum,
@@ -504,9 +515,10 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
   const int nseg = __builtin_amdgcn_readfirstlane(nseg_v);
   total = __builtin_amdgcn_readfirstlane(total);
   const int total_tok = total;  // keys of the active clusters; EAR appends the inactive centroids
+  const int ear_tile = (total_tok + kKT - 1) / kKT;  // EAR: first tile of centroids
   if constexpr (EAR) {
     const int ncent = build_centroids(mrow, ks + (size_t)b * kn, kn, cent_idx, cent_bias, red);
-    total = __builtin_amdgcn_readfirstlane(total_tok + ncent);
+    total = __builtin_amdgcn_readfirstlane(ncent > 0 ? ear_tile * kKT + ncent : total_tok);
   }
 
   if (total == 0) {
@@ -535,8 +547,8 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
 
   // Row tables (lane = tile position): in a full item wave 0 resolves K tiles and wave 1 V tiles; in a
   // half item waves 0 and 1 resolve stream 0 (even tiles), waves 2 and 3 stream 1 (odd tiles).
-  // Rows past the stream repeat its last token row (0 when an EAR row has no active tokens); EAR
-  // centroid j of the K (V) table is row crow_k + j (crow_v + j).
+  // Rows past the stream (and past an EAR stream's tokens in their last tile) repeat its last token row; the tables
+  // of EAR centroid tiles hold centroid indices.
   int last_row = nseg > 0 ? seg_start[nseg - 1] + (total_tok - 1 - seg_cum[nseg - 1]) : 0;
   if constexpr (IDX) last_row = kix[last_row];
   KvCursor cursor;
@@ -549,7 +561,6 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
   if constexpr (IDX) {
     if (resolver && p_first < total_tok) pend = kix[cursor_row(cursor, seg_start, seg_cum, p_first)];
   }
-  const int crow = (wave & 1) ? crow_v : crow_k;  // the resolving waves: even for K, odd for V
   // Table of tile t; the wave's next table is tile t + step (full items 1, half items 2).
   auto resolve = [&](int32_t* tab, int t, int step) __attribute__((always_inline)) {
     const int p = t * kKT + lane;
@@ -559,8 +570,8 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
       else
         tab[lane] = cursor_row(cursor, seg_start, seg_cum, p);
     }
-    else if (EAR && p < total)
-      tab[lane] = crow + cent_idx[p - total_tok];
+    else if (EAR && t >= ear_tile)
+      tab[lane] = cent_idx[max(0, min(p, total - 1) - ear_tile * kKT)];
     else
       tab[lane] = last_row;
     if constexpr (IDX) {
@@ -577,14 +588,9 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
 #pragma unroll
     for (int j = 0; j < kDmaIt; ++j) {
       const int r = 4 * (kDmaIt * wg + j) + prow;
-      if constexpr (EAR) {
-        // negative rows for EAR centroid rows below the token buffer
-        lds_dma16(src + (long long)rows[j] * 128 + swz(r, pch) * 8, buf + 4 * (kDmaIt * wg + j) * 128);
-      } else {
-        // a head's rows are < 2^24: a 32-bit byte offset from the wave-uniform base (SGPR-based addressing)
-        const uint32_t off = (uint32_t)rows[j] * 256u + (uint32_t)swz(r, pch) * 16u;
-        lds_dma16((const char*)src + off, buf + 4 * (kDmaIt * wg + j) * 128);
-      }
+      // a head's rows are < 2^24: a 32-bit byte offset from the wave-uniform base (SGPR-based addressing)
+      const uint32_t off = (uint32_t)rows[j] * 256u + (uint32_t)swz(r, pch) * 16u;
+      lds_dma16((const char*)src + off, buf + 4 * (kDmaIt * wg + j) * 128);
     }
   };
   // The same copies one group at a time (full items: interleaved with group B's softmax), with the
@@ -595,19 +601,16 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
   };
   auto dma_one = [&](const uint16_t* src, int row, int j, uint16_t* buf) __attribute__((always_inline)) {
     const int r = 4 * (kDmaIt * wg + j) + prow;
-    if constexpr (EAR) {
-      lds_dma16(src + (long long)row * 128 + swz(r, pch) * 8, buf + 4 * (kDmaIt * wg + j) * 128);
-    } else {
-      const uint32_t off = (uint32_t)row * 256u + (uint32_t)swz(r, pch) * 16u;
-      lds_dma16((const char*)src + off, buf + 4 * (kDmaIt * wg + j) * 128);
-    }
+    const uint32_t off = (uint32_t)row * 256u + (uint32_t)swz(r, pch) * 16u;
+    lds_dma16((const char*)src + off, buf + 4 * (kDmaIt * wg + j) * 128);
   };
-  auto dma_all = [&](int4 rk4, uint16_t* kdst, int4 rv4, uint16_t* vdst) __attribute__((always_inline)) {
+  auto dma_all = [&](const uint16_t* ksrc, int4 rk4, uint16_t* kdst, const uint16_t* vsrc, int4 rv4,
+                     uint16_t* vdst) __attribute__((always_inline)) {
     const int rka[4] = {rk4.x, rk4.y, rk4.z, rk4.w}, rva[4] = {rv4.x, rv4.y, rv4.z, rv4.w};
 #pragma unroll
-    for (int j = 0; j < kDmaIt; ++j) dma_one(kb, rka[j], j, kdst);
+    for (int j = 0; j < kDmaIt; ++j) dma_one(ksrc, rka[j], j, kdst);
 #pragma unroll
-    for (int j = 0; j < kDmaIt; ++j) dma_one(vb, rva[j], j, vdst);
+    for (int j = 0; j < kDmaIt; ++j) dma_one(vsrc, rva[j], j, vdst);
   };
 
   int koffs[8], voffs[2][4];
@@ -624,6 +627,23 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
   }
 
   const int ntiles = (total + kKT - 1) / kKT;
+  // Base of a tile's K (V) rows.  Past the stream: the tokens', with the rows of ear_rows.
+  auto ktile = [&](int t) __attribute__((always_inline)) -> const uint16_t* {
+    if constexpr (EAR) return uniform_ptr(t >= ear_tile && t < ntiles ? kcb : kb);
+    return kb;
+  };
+  auto vtile = [&](int t) __attribute__((always_inline)) -> const uint16_t* {
+    if constexpr (EAR) return uniform_ptr(t >= ear_tile && t < ntiles ? vcb : vb);
+    return vb;
+  };
+  // Rows of the copies of tile t from its table.  A tile past an EAR stream takes row 0 (its table may hold the rows
+  // of another buffer); otherwise the table's rows lie in the head whatever tile they are of.
+  auto trows = [&](const int32_t* tab, int t) __attribute__((always_inline)) -> int4 {
+    if constexpr (EAR) {
+      if (t >= ntiles) return make_int4(0, 0, 0, 0);
+    }
+    return dma_rows(tab);
+  };
   f32x16_t sacc[2];
   u32x4_t pop[2][2];
 
@@ -689,38 +709,34 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
   // VALU phase V(t): online softmax of S(t) -> bf16 P(t) (per lane: one query, 32 of 64 keys).  With
   // dmaon the eight copy groups of this wave (rows rk4 into kdst, rv4 into vdst) are issued between the
   // exponentials, one per four scores, so the vector-memory path sees them spread over the phase.
-  auto vphase = [&](int t, bool dmaon = false, int4 rk4 = int4{}, uint16_t* kdst = nullptr, int4 rv4 = int4{},
+  auto vphase = [&](int t, bool dmaon = false, const uint16_t* ksrc = nullptr, int4 rk4 = int4{},
+                    uint16_t* kdst = nullptr, const uint16_t* vsrc = nullptr, int4 rv4 = int4{},
                     uint16_t* vdst = nullptr) __attribute__((always_inline)) {
     // sl: the factor from sacc to log2-domain logits (1 once an EAR tile is pre-scaled and biased)
     float sl = scale_log2;
     if constexpr (EAR) {
-      if ((t + 1) * kKT > total_tok) {
-        const int tbase = t * kKT;
+      if (t >= ear_tile) {  // a tile of centroids: their biases, -inf past the last one
+        const float* cb = cent_bias + (t - ear_tile) * kKT + h * 4;
 #pragma unroll
         for (int kb2 = 0; kb2 < 2; ++kb2)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int p = tbase + kb2 * 32 + (r / 4) * 8 + h * 4 + (r % 4);
-            float xv = sacc[kb2][r] * scale_log2;
-            if (p >= total)
-              xv = -INFINITY;
-            else if (p >= total_tok)
-              xv += cent_bias[p - total_tok];
-            sacc[kb2][r] = xv;
+          for (int r4 = 0; r4 < 4; ++r4) {
+            const f32x4_t bias = *(const f32x4_t*)(cb + kb2 * 32 + r4 * 8);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sacc[kb2][4 * r4 + e] = fmaf(sacc[kb2][4 * r4 + e], scale_log2, bias[e]);
           }
         sl = 1.0f;
       }
-    } else {
-      if ((t + 1) * kKT > total) {
-        const int tbase = t * kKT;
+    }
+    if ((t + 1) * kKT > total_tok && (!EAR || t < ear_tile)) {
+      const int tbase = t * kKT;
 #pragma unroll
-        for (int kb2 = 0; kb2 < 2; ++kb2)
+      for (int kb2 = 0; kb2 < 2; ++kb2)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int key = kb2 * 32 + (r / 4) * 8 + h * 4 + (r % 4);
-            if (tbase + key >= total) sacc[kb2][r] = -INFINITY;
-          }
-      }
+        for (int r = 0; r < 16; ++r) {
+          const int key = kb2 * 32 + (r / 4) * 8 + h * 4 + (r % 4);
+          if (tbase + key >= total_tok) sacc[kb2][r] = -INFINITY;
+        }
     }
     // P against the running max m_run.  The lane's row sum over its 32 values bounds each of them, so
     // the maximum is only needed when the sum leaves [0, 2^13]: a value more than 13 (log2) above
@@ -741,9 +757,9 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
             const int j = (kb2 * 16 + r) / 4;
             __builtin_amdgcn_sched_group_barrier(0x002, 12, 0);
             if (j < kDmaIt)
-              dma_one(kb, rka[j], j, kdst);
+              dma_one(ksrc, rka[j], j, kdst);
             else
-              dma_one(vb, rva[j - kDmaIt], j - kDmaIt, vdst);
+              dma_one(vsrc, rva[j - kDmaIt], j - kDmaIt, vdst);
             __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
           }
         }
@@ -838,15 +854,30 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
     mm(15);
   };
   // Softmax of the chunk of tile t; the eight copies of a copying wave go out one per two exponentials.
-  // Only called for a chunk that holds a key (so the running maximum is finite after the first call).
-  auto vphase_q = [&](int t, bool dmaon = false, int4 rk4 = int4{}, uint16_t* kdst = nullptr, int4 rv4 = int4{},
+  // Only called for a chunk that holds a key (so the running maximum is finite after the first call); the second
+  // half of an EAR stream's last token tile can be empty, so there the maximum has a floor.
+  auto vphase_q = [&](int t, bool dmaon = false, const uint16_t* ksrc = nullptr, int4 rk4 = int4{},
+                      uint16_t* kdst = nullptr, const uint16_t* vsrc = nullptr, int4 rv4 = int4{},
                       uint16_t* vdst = nullptr) __attribute__((always_inline)) {
     const int tbase = t * kKT + chunk * 32;
-    if (tbase + 32 > total) {
+    float sl = scale_log2;
+    if constexpr (EAR) {
+      if (t >= ear_tile) {
+        const float* cb = cent_bias + (t - ear_tile) * kKT + chunk * 32 + h * 4;
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+          const f32x4_t bias = *(const f32x4_t*)(cb + r4 * 8);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sacc[0][4 * r4 + e] = fmaf(sacc[0][4 * r4 + e], scale_log2, bias[e]);
+        }
+        sl = 1.0f;
+      }
+    }
+    if (tbase + 32 > total_tok && (!EAR || t < ear_tile)) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int key = (r / 4) * 8 + h * 4 + (r % 4);
-        if (tbase + key >= total) sacc[0][r] = -INFINITY;
+        if (tbase + key >= total_tok) sacc[0][r] = -INFINITY;
       }
     }
     auto pexp = [&](bool dm) __attribute__((always_inline)) -> float {
@@ -856,14 +887,14 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
       float pv[16];
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        pv[r] = __builtin_amdgcn_exp2f(fmaf(sacc[0][r], scale_log2, mneg));
+        pv[r] = __builtin_amdgcn_exp2f(fmaf(sacc[0][r], sl, mneg));
         if (dm && r % 2 == 1) {
           const int j = r / 2;
           __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
           if (j < kDmaIt)
-            dma_one(kb, rka[j], j, kdst);
+            dma_one(ksrc, rka[j], j, kdst);
           else
-            dma_one(vb, rva[j - kDmaIt], j - kDmaIt, vdst);
+            dma_one(vsrc, rva[j - kDmaIt], j - kDmaIt, vdst);
           __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
         }
       }
@@ -880,8 +911,8 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
       float mx = sacc[0][0];
 #pragma unroll
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sacc[0][r]);
-      mx = xhalf_max(mx) * scale_log2;
-      const float m_new = fmaxf(m_run, mx);
+      mx = xhalf_max(mx) * sl;
+      const float m_new = fmaxf(m_run, EAR ? fmaxf(mx, -3.0e38f) : mx);
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
       m_run = m_new;
       l_run *= alpha;
@@ -904,9 +935,9 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
       constexpr int rw0 = kB ? 4 : 0, rw1 = kB ? 5 : 1;  // the resolving waves
       auto bvph = [&](int t, int4 rk4, uint16_t* kdst, int4 rv4, uint16_t* vdst) __attribute__((always_inline)) {
         if constexpr (kB)
-          vphase_q(t, true, rk4, kdst, rv4, vdst);
+          vphase_q(t, true, ktile(t + 2), rk4, kdst, vtile(t + 1), rv4, vdst);
         else
-          vphase(t, true, rk4, kdst, rv4, vdst);
+          vphase(t, true, ktile(t + 2), rk4, kdst, vtile(t + 1), rv4, vdst);
       };
       auto bmph = [&](const uint16_t* vt, const uint16_t* knext) __attribute__((always_inline)) {
         if constexpr (kB)
@@ -928,9 +959,9 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
       }
       __syncthreads();
       if (group_b) {
-        dma(kb, rowtab[0][0][0], k_s0);
-        dma(vb, rowtab[0][1][0], v_s0);
-        if (ntiles > 1) dma(kb, rowtab[0][0][1], k_s1);
+        dma(ktile(0), rowtab[0][0][0], k_s0);
+        dma(vtile(0), rowtab[0][1][0], v_s0);
+        if (ntiles > 1) dma(ktile(1), rowtab[0][0][1], k_s1);
         __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
       __syncthreads();
@@ -955,8 +986,8 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
       __syncthreads();
       int4 rk = make_int4(0, 0, 0, 0), rv = make_int4(0, 0, 0, 0);
       if (group_b) {
-        rk = dma_rows(rowtab[0][0][0]);
-        rv = dma_rows(rowtab[0][1][1]);
+        rk = trows(rowtab[0][0][0], 2);
+        rv = trows(rowtab[0][1][1], 1);
       }
 
       // Half-steps h = 0 .. 2T-1 (unrolled by 4: tile parity fixes the buffers).
@@ -972,7 +1003,7 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
           if (active && (!kB || t < nvb))
             bvph(t, rk, k_s0, rv, v_s1);
           else
-            dma_all(rk, k_s0, rv, v_s1);
+            dma_all(ktile(t + 2), rk, k_s0, vtile(t + 1), rv, v_s1);
         }
         __syncthreads();
         if (!group_b) {
@@ -987,8 +1018,8 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
             if (wave == 4 && t + 4 < ntiles) resolve(rowtab[0][0][t & 1], t + 4, 1);
             if (wave == 5 && t + 3 < ntiles) resolve(rowtab[0][1][(t + 1) & 1], t + 3, 1);
           }
-          rk = dma_rows(rowtab[0][0][(t + 1) & 1]);
-          rv = dma_rows(rowtab[0][1][t & 1]);
+          rk = trows(rowtab[0][0][(t + 1) & 1], t + 3);
+          rv = trows(rowtab[0][1][t & 1], t + 2);
           __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
         __syncthreads();
@@ -1000,7 +1031,7 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
           if (active && (!kB || t + 1 < nvb))
             bvph(t + 1, rk, k_s1, rv, v_s0);
           else
-            dma_all(rk, k_s1, rv, v_s0);
+            dma_all(ktile(t + 3), rk, k_s1, vtile(t + 2), rv, v_s0);
         }
         __syncthreads();
         if (!group_b) {
@@ -1015,8 +1046,8 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
             if (wave == 4 && t + 5 < ntiles) resolve(rowtab[0][0][(t + 1) & 1], t + 5, 1);
             if (wave == 5 && t + 4 < ntiles) resolve(rowtab[0][1][t & 1], t + 4, 1);
           }
-          rk = dma_rows(rowtab[0][0][t & 1]);
-          rv = dma_rows(rowtab[0][1][(t + 1) & 1]);
+          rk = trows(rowtab[0][0][t & 1], t + 4);
+          rv = trows(rowtab[0][1][(t + 1) & 1], t + 3);
           __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
         __syncthreads();
@@ -1095,13 +1126,13 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
     }
     __syncthreads();
     if (group_b) {
-      dma(kb, rowtab[0][0][0], k_s0);
-      dma(vb, rowtab[0][1][0], v_s0);
-      if (n0 > 1) dma(kb, rowtab[0][0][1], k_s1);
+      dma(ktile(0), rowtab[0][0][0], k_s0);
+      dma(vtile(0), rowtab[0][1][0], v_s0);
+      if (n0 > 1) dma(ktile(2), rowtab[0][0][1], k_s1);
       if (n1 > 0) {
-        dma(kb, rowtab[1][0][0], k1_s0);
-        dma(vb, rowtab[1][1][0], v1_s0);
-        if (n1 > 1) dma(kb, rowtab[1][0][1], k1_s1);
+        dma(ktile(1), rowtab[1][0][0], k1_s0);
+        dma(vtile(1), rowtab[1][1][0], v1_s0);
+        if (n1 > 1) dma(ktile(3), rowtab[1][0][1], k1_s1);
       }
       __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
@@ -1129,17 +1160,17 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
       } else {
         rows2(1, u, n1, rk, rv);
         if (active && u < n1)
-          vphase(2 * u + 1, true, rk, k1_s0, rv, v1_s1);
+          vphase(2 * u + 1, true, ktile(2 * u + 5), rk, k1_s0, vtile(2 * u + 3), rv, v1_s1);
         else
-          dma_all(rk, k1_s0, rv, v1_s1);
+          dma_all(ktile(2 * u + 5), rk, k1_s0, vtile(2 * u + 3), rv, v1_s1);
       }
       __syncthreads();
       if (!group_b) {
         rows2(0, u, n0, rk, rv);
         if (active && u + 1 < n0)
-          vphase(2 * u + 2, true, rk, k_s0, rv, v_s1);
+          vphase(2 * u + 2, true, ktile(2 * u + 4), rk, k_s0, vtile(2 * u + 2), rv, v_s1);
         else
-          dma_all(rk, k_s0, rv, v_s1);
+          dma_all(ktile(2 * u + 4), rk, k_s0, vtile(2 * u + 2), rv, v_s1);
       } else {
         if (active && u < n1) mphase(u, v1_s0, k1_s1);
       }
@@ -1151,17 +1182,17 @@ __global__ void __launch_bounds__(kVWaves * kWave) __attribute__((amdgpu_waves_p
       } else {
         rows2(1, u + 1, n1, rk, rv);
         if (active && u + 1 < n1)
-          vphase(2 * u + 3, true, rk, k1_s1, rv, v1_s0);
+          vphase(2 * u + 3, true, ktile(2 * u + 7), rk, k1_s1, vtile(2 * u + 5), rv, v1_s0);
         else
-          dma_all(rk, k1_s1, rv, v1_s0);
+          dma_all(ktile(2 * u + 7), rk, k1_s1, vtile(2 * u + 5), rv, v1_s0);
       }
       __syncthreads();
       if (!group_b) {
         rows2(0, u + 1, n0, rk, rv);
         if (active && u + 2 < n0)
-          vphase(2 * u + 4, true, rk, k_s1, rv, v_s0);
+          vphase(2 * u + 4, true, ktile(2 * u + 6), rk, k_s1, vtile(2 * u + 4), rv, v_s0);
         else
-          dma_all(rk, k_s1, rv, v_s0);
+          dma_all(ktile(2 * u + 6), rk, k_s1, vtile(2 * u + 4), rv, v_s0);
       } else {
         if (active && u + 1 < n1) mphase(u + 1, v1_s1, k1_s0);
       }
@@ -1305,7 +1336,7 @@ int vbsa_launch(const char* name, const uint16_t* q, const uint16_t* k, const ui
   SVOO_REQUIRE(workspace && ws_bytes >= lay.total, SVOO_ERR_WORKSPACE, "%s: workspace %zu < %zu", name, ws_bytes,
                lay.total);
   if (EAR) {
-    // centroid rows are addressed as signed int32 row offsets from the token buffers
+    // the entry's contract on where the centroid buffers lie
     const long long dk = (long long)(uintptr_t)kc - (long long)(uintptr_t)k;
     const long long dv = (long long)(uintptr_t)vc - (long long)(uintptr_t)v;
     SVOO_REQUIRE(dk % 256 == 0 && dv % 256 == 0, SVOO_ERR_INVALID_ARG,
@@ -1323,11 +1354,10 @@ int vbsa_launch(const char* name, const uint16_t* q, const uint16_t* k, const ui
   int32_t* work = (int32_t*)(base + lay.work);
   int32_t* list = (int32_t*)(base + lay.list);
   constexpr int qtile = VbsaCfg<kDefaultQB>::kQTile;
-  const size_t smem = (size_t)((EAR ? 4 : 2) * kn + 1) * sizeof(int32_t);
+  const size_t smem = (size_t)(2 * kn + 1 + (EAR ? kn + (kn + kKT - 1) / kKT * kKT : 0)) * sizeof(int32_t);
   // Half items need the kernel with a second set of K/V buffers (130 KB of static LDS with the row
-  // tables), which leaves 28 KB of the 160 KB LDS for the segment tables.  The EAR kernel (64-bit copy
-  // addresses for the centroid rows) runs full items only: with both paths it exceeds 256 registers.
-  const bool half_ok = !EAR && smem <= (size_t)28 * 1024;
+  // tables), which leaves 28 KB of the 160 KB LDS for the segment tables.
+  const bool half_ok = smem <= (size_t)28 * 1024;
   hipLaunchKernelGGL(vbsa_plan_kernel, dim3(bh), dim3(kPlanThreads), 0, st, q_sizes, k_sizes, map, EAR ? 1 : 0, work,
                      s, qn, kn, qtile, lay.cap, half_ok ? 1 : 0, qoff, koff, items, nitems, status);
   if (int rc = check_launch(name)) return rc;
@@ -1338,8 +1368,8 @@ int vbsa_launch(const char* name, const uint16_t* q, const uint16_t* k, const ui
   const long long nblocks = (total_items + 8 * kXcdRun - 1) / (8 * kXcdRun) * (8 * kXcdRun);
   SVOO_REQUIRE(nblocks < (1ll << 31), SVOO_ERR_UNSUPPORTED, "%s: too many work items", name);
   const float scale_log2 = (float)(1.4426950408889634 / sqrt((double)d));
-  if (!EAR && half_ok)
-    hipLaunchKernelGGL((vbsa_attn_kernel<kDefaultQB, EAR, IDX, !EAR>), dim3((unsigned)nblocks), dim3(kVWaves * kWave),
+  if (half_ok)
+    hipLaunchKernelGGL((vbsa_attn_kernel<kDefaultQB, EAR, IDX, true>), dim3((unsigned)nblocks), dim3(kVWaves * kWave),
                        smem, st, q, k, v, kc, vc, map, k_sizes, o, s, qn, kn, lay.cap, total_items, qoff, koff, items,
                        nitems, scale_log2, q_idx, k_idx, heads, list);
   else

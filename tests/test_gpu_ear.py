@@ -207,6 +207,39 @@ def test_compensated_attention_matches_oracle(gpu, h, qn, kn, s, density, seed):
     _attn_check(out, O.ear_compensated_attention(q, k, v, kc, vc, m, qs, ks))
 
 
+@pytest.mark.parametrize("extra", [0, 57, 64, 75])
+def test_compensated_attention_at_stream_and_item_edges(gpu, extra):
+    """Query clusters of every item kind (half, split between the groups, full, full with each as the last tile) over
+    streams whose token part ends at, before and after a tile or half a tile, with 0 .. 83 centroids behind it (none,
+    one tile, just above one): the streams' token part is padded to whole tiles."""
+    from svoo_amd.ear import dynamic_block_sparse_prune_fwd
+
+    totals = (0, 1, 31, 32, 33, 63, 64, 65, 96, 97, 128, 129, 255)
+    sizes = (64, 128, 129, 192, 193, 256, 300, 386, 449)
+    say("ear attention, stream and item edges", extra)
+    bits = [1 << e for e in range(8)]  # a row's token total is the sum of the clusters it takes
+    qs = [sizes[i % len(sizes)] for i in range(2 * len(totals))]
+    s = sum(qs)
+    rest = s - sum(bits)
+    ks = bits + ([rest // extra + (1 if j < rest % extra else 0) for j in range(extra)] if extra else [rest])
+    kn = len(ks)
+    m = np.zeros((1, 1, len(qs), kn), bool)
+    for i in range(len(qs)):
+        t = totals[i % len(totals)]
+        m[0, 0, i, :8] = [(t >> e) & 1 for e in range(8)]
+        if extra == 0:
+            m[0, 0, i, 8] = i % 3 == 0  # the one large cluster: sometimes every cluster but a few is active
+    qs, ks = np.asarray(qs, np.int32)[None, None], np.asarray(ks, np.int32)[None, None]
+    q, qt = rand_bf16((1, 1, s, 128), 31, gpu, 0.5)
+    k, kt = rand_bf16((1, 1, s, 128), 32, gpu, 0.5)
+    v, vt = rand_bf16((1, 1, s, 128), 33, gpu)
+    kc, kct = rand_bf16((1, 1, kn, 128), 34, gpu, 0.5)
+    vc, vct = rand_bf16((1, 1, kn, 128), 35, gpu)
+    out = dynamic_block_sparse_prune_fwd(qt, kt, vt, kct, vct, torch.from_numpy(m).to(gpu), _i32(qs, gpu),
+                                         _i32(ks, gpu))
+    _attn_check(out, O.ear_compensated_attention(q, k, v, kc, vc, m, qs, ks))
+
+
 def test_compensation_of_point_mass_clusters_is_dense(gpu):
     from svoo_amd.ear import dynamic_block_sparse_prune_fwd
 
