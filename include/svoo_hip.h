@@ -105,6 +105,23 @@ int svoo_convert_rows(const void* src, int src_type, int src_cols, void* dst, in
                       long long rows, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
+ * Projected rows to attention heads: q, k, v rows of H*D bf16 elements (row strides in elements, rows at 16-byte
+ * addresses) to [H][out_rows][D] buffers, rows out_row0 .. out_row0 + rows - 1.  D is 64 or 128, H*D <= 8192.
+ *   norm: 0 none; 1 RMSNorm of q and k over the row, 2 over each head, y = bf16(w * (x * rsqrt(mean(x^2) + eps))) in
+ *     fp32 (q_weight / k_weight bf16 or NULL for ones; rows at 16-byte addresses);
+ *   cos_table / sin_table: fp32 [rope_rows][D] or NULL; rows below rope_rows of q and k are rotated on interleaved pairs,
+ *     y0 = x0 c0 - x1 s0, y1 = x1 c1 + x0 s1, products rounded to fp32; rope_form 0 takes c0 = c1 = the pair's even
+ *     cosine and s0 = s1 = its odd sine, 1 each element's own.
+ * Replaces the norm, _apply_rotary_emb and transposes of svoo/models/wan/attention.py:153-215 and of
+ * svoo/models/hunyuan10/attention.py:305-353, 536-575.
+ * ------------------------------------------------------------------------------------------- */
+int svoo_qkv_heads(const uint16_t* q, const uint16_t* k, const uint16_t* v, long long q_stride, long long k_stride,
+                   long long v_stride, uint16_t* q_out, uint16_t* k_out, uint16_t* v_out, int rows, int heads, int d,
+                   int out_rows, int out_row0, int norm, const uint16_t* q_weight, const uint16_t* k_weight,
+                   float q_eps, float k_eps, const float* cos_table, const float* sin_table, int rope_rows,
+                   int rope_form, void* stream);
+
+/* ---------------------------------------------------------------------------------------------
  * Co-clustering (profile-space k-means).
  *   svoo_cocluster_prep: P = l2norm(bf16(A B^T)) ([BH][J][KP], optional output), E = P B split into
  *     E_hi = bf16(E), E_lo = bf16(E - E_hi), both [BH][jpad][D]; rows J..jpad-1 repeat row J-1.

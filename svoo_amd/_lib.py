@@ -54,6 +54,8 @@ _SIGS = {
     "svoo_ear_efficiency": (c_int, [P, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_float, c_float,
                                     P, P]),
     "svoo_ear_select": (c_int, [P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_float, P, P]),
+    "svoo_qkv_heads": (c_int, [P, P, P, c_longlong, c_longlong, c_longlong, P, P, P, c_int, c_int, c_int, c_int, c_int,
+                               c_int, P, P, c_float, c_float, P, P, c_int, c_int, P]),
     "svoo_vbsa_ear_fwd": (c_int, [P, P, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, P, c_size_t, P, P]),
 }
 

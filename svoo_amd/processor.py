@@ -33,7 +33,7 @@ from .ear import dynamic_block_sparse_prune_fwd, ear_map_and_value_centroids
 from .sparsity.exact import (compute_exact_attention_sparsity, format_sparsity_log, has_completed_sparsity_entry,
                              record_sparsity_entry)
 from .permute import apply_inverse_permutation, apply_inverse_permutation_bshd, permute_pair_by_indices
-from . import _lib
+from . import _lib, heads
 
 
 def _env_on(name: str) -> bool:
@@ -190,6 +190,44 @@ class WanAttn_SAPAttn_Processor:
         return (query.transpose(1, 2).contiguous(), key.transpose(1, 2).contiguous(),
                 value.transpose(1, 2).contiguous())
 
+    def _uses_own(self, base, *names) -> bool:
+        """The methods ``names`` are ``base``'s own: no subclass or instance replaced one."""
+        return all(n not in self.__dict__ and getattr(type(self), n) is getattr(base, n) for n in names)
+
+    def _qkv_heads(self, attn, query, key, value, rotary_emb):
+        """Norm, RoPE and transposition of projected self-attention ``[1, S, H*D]`` tensors in one HIP pass, or None
+        where the separate operations have to run (the same values but for the norm's order of summation).  Norm
+        modules other than ``torch.nn.RMSNorm`` are called first."""
+        h = attn.heads
+        if not (self._uses_own(WanAttn_SAPAttn_Processor, "get_qk_norm", "get_transpose_qkv")
+                and heads.plain_execution() and all(heads.rows_ok(t, h) for t in (query, key, value))
+                and query.shape == key.shape == value.shape):
+            return None
+        s, dim = query.shape[1:]
+        if rotary_emb is not None and not heads.tables_ok(rotary_emb, (1, s, 1, dim // h), query.device):
+            return None
+        norms = [getattr(attn, n, None) for n in ("norm_q", "norm_k")]
+        kw = {}
+        if norms[0] is not None or norms[1] is not None:
+            params = [heads.rms_norm_params(n, dim, query.device) for n in norms]
+            if None not in params:
+                kw = dict(norm=1, q_norm=params[0], k_norm=params[1])
+            else:
+                query, key = self.get_qk_norm(attn, query, key)
+                if not (heads.rows_ok(query, h) and heads.rows_ok(key, h) and query.shape == key.shape == value.shape):
+                    return self._qkv_separately(attn, query, key, value, rotary_emb)
+        if rotary_emb is not None:
+            kw.update(rope=rotary_emb, rope_rows=s)
+        return heads.qkv_heads(query, key, value, h, **kw)
+
+    def _qkv_separately(self, attn, query, key, value, rotary_emb):
+        """The operations after the norms: heads, RoPE, transposition."""
+        query, key, value = (t.unflatten(2, (attn.heads, -1)) for t in (query, key, value))
+        if rotary_emb is not None:
+            query = _apply_rotary_emb(query, *rotary_emb)
+            key = _apply_rotary_emb(key, *rotary_emb)
+        return self.get_transpose_qkv(attn, query, key, value)
+
     def get_o(self, attn, query, hidden_states, hidden_states_img):
         if hidden_states.dim() == 4:
             hidden_states = hidden_states.transpose(1, 2).flatten(2, 3)
@@ -211,14 +249,11 @@ class WanAttn_SAPAttn_Processor:
             encoder_hidden_states_img = encoder_hidden_states[:, :image_context_length]
             encoder_hidden_states = encoder_hidden_states[:, image_context_length:]
         query, key, value = self.get_qkv(attn, hidden_states, encoder_hidden_states)
-        query, key = self.get_qk_norm(attn, query, key)
-        query = query.unflatten(2, (attn.heads, -1))
-        key = key.unflatten(2, (attn.heads, -1))
-        value = value.unflatten(2, (attn.heads, -1))
-        if rotary_emb is not None:
-            query = _apply_rotary_emb(query, *rotary_emb)
-            key = _apply_rotary_emb(key, *rotary_emb)
-        query, key, value = self.get_transpose_qkv(attn, query, key, value)
+        fused = self._qkv_heads(attn, query, key, value, rotary_emb)
+        if fused is None:
+            query, key = self.get_qk_norm(attn, query, key)
+            fused = self._qkv_separately(attn, query, key, value, rotary_emb)
+        query, key, value = fused
 
         hidden_states_img = None
         if encoder_hidden_states_img is not None:
@@ -608,6 +643,52 @@ class Hunyuan_SAPAttn_Processor(WanAttn_SAPAttn_Processor):
             value = torch.cat([value, ev], dim=2)
         return query.contiguous(), key.contiguous(), value.contiguous()
 
+    def _joint_heads(self, attn, query, key, value, encoder_hidden_states, image_rotary_emb):
+        """Norm, RoPE and transposition of projected ``[1, S, H*D]`` tensors, and of a double-stream block's text
+        projections behind them, in one HIP pass each; None where the separate operations have to run."""
+        h = attn.heads
+        if not (self._uses_own(Hunyuan_SAPAttn_Processor, "get_qk_norm", "get_transpose_qkv", "get_rotary_emb",
+                               "get_encoder_condition_and_concat")
+                and heads.plain_execution() and all(heads.rows_ok(t, h) for t in (query, key, value))
+                and query.shape == key.shape == value.shape):
+            return None
+        s, dim = query.shape[1:]
+        d = dim // h
+        double = getattr(attn, "add_q_proj", None) is not None and encoder_hidden_states is not None
+        text = encoder_hidden_states.shape[1] if encoder_hidden_states is not None else 0
+        video = s if double else s - text
+        kw = {}
+        if image_rotary_emb is not None:
+            # a text of no tokens would make the reference's slices [:-0] empty: its operations decide
+            if (text == 0 and encoder_hidden_states is not None) or video <= 0 or \
+                    not heads.tables_ok(image_rotary_emb, (video, d), query.device):
+                return None
+            kw.update(rope=image_rotary_emb, rope_rows=video, per_element=True)
+
+        def norm_args(names):
+            mods = [getattr(attn, n, None) for n in names]
+            if mods[0] is None and mods[1] is None:
+                return {}
+            params = [heads.rms_norm_params(m, d, query.device) for m in mods]
+            return None if None in params else dict(norm=2, q_norm=params[0], k_norm=params[1])
+
+        norm = norm_args(("norm_q", "norm_k"))
+        if norm is None:
+            return None
+        if not double:
+            return heads.qkv_heads(query, key, value, h, **norm, **kw)
+        # the text's keys are normed where its queries are (get_encoder_condition_and_concat)
+        text_norm = norm_args(("norm_added_q", "norm_added_k")) if getattr(attn, "norm_added_q", None) is not None else {}
+        if text_norm is None or text <= 0:
+            return None
+        projections = [getattr(attn, n, None) for n in ("add_q_proj", "add_k_proj", "add_v_proj")]
+        if not all(heads.linear_ok(p, encoder_hidden_states, dim) for p in projections):
+            return None
+        added = tuple(p(encoder_hidden_states) for p in projections)
+        out = tuple(torch.empty(1, h, s + text, d, dtype=query.dtype, device=query.device) for _ in range(3))
+        heads.qkv_heads(query, key, value, h, out=out, **norm, **kw)
+        return heads.qkv_heads(*added, h, out=out, out_row0=s, **text_norm)
+
     def get_cu_max_seqlen(self, attention_mask, device):
         """``([0, valid, total]`` for q and kv, max lengths); built on the device (no host read-back)."""
         mask = attention_mask.to(device)
@@ -634,10 +715,14 @@ class Hunyuan_SAPAttn_Processor(WanAttn_SAPAttn_Processor):
         if getattr(attn, "add_q_proj", None) is None and encoder_hidden_states is not None:
             hidden_states = torch.cat([hidden_states, encoder_hidden_states], dim=1)
         query, key, value = self.get_qkv(attn, hidden_states)
-        query, key, value = self.get_transpose_qkv(attn, query, key, value)
-        query, key = self.get_qk_norm(attn, query, key)
-        query, key = self.get_rotary_emb(attn, query, key, image_rotary_emb, encoder_hidden_states)
-        query, key, value = self.get_encoder_condition_and_concat(attn, query, key, value, encoder_hidden_states)
+        fused = self._joint_heads(attn, query, key, value, encoder_hidden_states, image_rotary_emb)
+        if fused is not None:
+            query, key, value = fused
+        else:
+            query, key, value = self.get_transpose_qkv(attn, query, key, value)
+            query, key = self.get_qk_norm(attn, query, key)
+            query, key = self.get_rotary_emb(attn, query, key, image_rotary_emb, encoder_hidden_states)
+            query, key, value = self.get_encoder_condition_and_concat(attn, query, key, value, encoder_hidden_states)
         if attention_mask is None:
             attention_mask = torch.ones(query.shape[2], dtype=torch.bool, device=query.device)
         cu_max_seqlens = self.get_cu_max_seqlen(attention_mask, query.device)
@@ -718,10 +803,8 @@ class Hunyuan_SAPAttn_Processor(WanAttn_SAPAttn_Processor):
 
         # 1. Video part: cluster (or reuse), per-head ratios, block mask.
         self._mark("start")
-        q_video = query[:, :, :video_length].contiguous()
-        k_video = key[:, :, :video_length].contiguous()
-        r = self.kmeans_clustering(q_video, k_video, self.layer_idx)
-        del q_video, k_video
+        # (views: a step that reuses the clustering reads neither, one that clusters makes them contiguous)
+        r = self.kmeans_clustering(query[:, :, :video_length], key[:, :, :video_length], self.layer_idx)
         self._mark("cluster")
         min_kc_ratio = self._get_min_kc_ratio_for_heads_from_step(self.current_inference_step, num_heads)
         q_sizes = r["qsizes"].view(cfg, num_heads, self.num_q_centroids)

@@ -1,0 +1,164 @@
+"""The one-pass norm + RoPE + transposition of the processors' projections (``svoo_qkv_heads``) against the separate
+tensor operations it stands in for, and the cases in which those have to run."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print("[case]", *a, flush=True)
+
+
+class Layer(torch.nn.Module):
+    """Projections and norms under the names the processors read."""
+
+    def __init__(self, heads, d, norm_width, gpu, double=False, fused=False):
+        super().__init__()
+        dim = heads * d
+        kw = dict(dtype=torch.bfloat16, device=gpu)
+        self.heads = heads
+        self.fused_projections = fused
+        if fused:
+            self.to_qkv = torch.nn.Linear(dim, 3 * dim, **kw)
+            self.cross_attention_dim_head = None
+        names = [] if fused else ["to_q", "to_k", "to_v"]
+        norms = ["norm_q", "norm_k"]
+        if double:
+            names += ["add_q_proj", "add_k_proj", "add_v_proj"]
+            norms += ["norm_added_q", "norm_added_k"]
+        for n in names:
+            setattr(self, n, torch.nn.Linear(dim, dim, **kw))
+        for n in norms:
+            m = torch.nn.RMSNorm(norm_width, eps=1e-6, **kw)
+            torch.nn.init.uniform_(m.weight, 0.5, 1.5)
+            setattr(self, n, m)
+        self.requires_grad_(False)
+
+
+def _tables(rows, d, gpu):
+    ang = torch.rand(rows, d, device=gpu) * 6.0  # each element its own angle: the forms differ in which they take
+    return ang.cos(), ang.sin()
+
+
+def _processor(base):
+    """A processor whose attention hands back the heads it was given."""
+
+    class P(base):
+        def attention_core_logic(self, query, key, value, *a):
+            self.got = (query, key, value)
+            return query if base.__name__.startswith("Hunyuan") else query.transpose(1, 2).flatten(2, 3)
+
+        def get_o(self, *a):
+            return None
+
+    return P(layer_idx=0)
+
+
+def _heads(proc, layer, x, separate, monkeypatch, **kw):
+    from svoo_amd import _lib, heads
+
+    calls = []
+    real = _lib.call
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "call", lambda name, *a: (calls.append(name), real(name, *a))[1])
+        if separate:
+            m.setattr(heads, "plain_execution", lambda: False)
+        proc(layer, x, timestep=torch.zeros(1), **kw)
+    assert all(t.is_contiguous() for t in proc.got)
+    return [t.clone() for t in proc.got], calls.count("svoo_qkv_heads")
+
+
+def _close(got, want):
+    """The norm's sums may round differently in another order: rstd moves by a few 2^-24, so a normed element moves by
+    at most one bf16 step (2^-8 of it) and a rotated pair by 2^-8 (|x0| + |x1|) and its own rounding."""
+    for g, w in zip(got, want):
+        g, w = g.double(), w.double()
+        pair = w.unflatten(-1, (-1, 2)).abs().sum(-1, keepdim=True).expand(*w.shape[:-1], w.shape[-1] // 2, 2).flatten(-2)
+        assert ((g - w).abs() <= 2.0 ** -6 * pair + 1e-30).all()
+        assert (g != w).double().mean() < 1e-2
+
+
+@pytest.mark.parametrize("heads,d,s,fused", [(12, 128, 333, False), (2, 128, 5, True), (5, 64, 130, False),
+                                             (40, 128, 65, False), (64, 128, 3, False), (1, 64, 1, False)])
+def test_wan_heads_equal_the_operations(gpu, monkeypatch, heads, d, s, fused):
+    from svoo_amd.processor import WanAttn_SAPAttn_Processor
+
+    say("wan heads", heads, d, s, fused)
+    torch.manual_seed(heads * s)
+    layer = Layer(heads, d, heads * d, gpu, fused=fused)
+    x = torch.randn(1, s, heads * d, device=gpu, dtype=torch.bfloat16)
+    proc = _processor(WanAttn_SAPAttn_Processor)
+    cos, sin = _tables(s, d, gpu)
+    kw = dict(rotary_emb=(cos[None, :, None], sin[None, :, None]))
+    want, n0 = _heads(proc, layer, x, True, monkeypatch, **kw)
+    got, n1 = _heads(proc, layer, x, False, monkeypatch, **kw)
+    assert (n0, n1) == (0, 1)
+    _close(got[:2], want[:2])
+    assert torch.equal(got[2], want[2])
+    # without the norm in the pass (another norm module) every bit is the operations'
+    layer.norm_q, layer.norm_k = torch.nn.Identity(), torch.nn.Identity()
+    for kw2 in (kw, {}):
+        want, _ = _heads(proc, layer, x, True, monkeypatch, **kw2)
+        got, n1 = _heads(proc, layer, x, False, monkeypatch, **kw2)
+        assert n1 == 1 and all(torch.equal(g, w) for g, w in zip(got, want))
+
+
+@pytest.mark.parametrize("double", [False, True])
+@pytest.mark.parametrize("heads,d,s,text", [(24, 128, 200, 33), (3, 64, 7, 1)])
+def test_hunyuan_heads_equal_the_operations(gpu, monkeypatch, heads, d, s, text, double):
+    from svoo_amd.processor import Hunyuan_SAPAttn_Processor
+
+    say("hunyuan heads", heads, d, s, text, double)
+    torch.manual_seed(s + text)
+    layer = Layer(heads, d, d, gpu, double=double)
+    x = torch.randn(1, s, heads * d, device=gpu, dtype=torch.bfloat16)
+    txt = torch.randn(1, text, heads * d, device=gpu, dtype=torch.bfloat16)
+    proc = _processor(Hunyuan_SAPAttn_Processor)
+    for kw in (dict(encoder_hidden_states=txt, image_rotary_emb=_tables(s, d, gpu)),
+               dict(encoder_hidden_states=txt), dict(image_rotary_emb=_tables(s, d, gpu))):
+        want, n0 = _heads(proc, layer, x, True, monkeypatch, **kw)
+        got, n1 = _heads(proc, layer, x, False, monkeypatch, **kw)
+        assert n0 == 0 and n1 == (2 if double and "encoder_hidden_states" in kw else 1)
+        _close(got[:2], want[:2])
+        assert torch.equal(got[2], want[2])
+
+
+def test_the_operations_run_where_the_pass_cannot(gpu, monkeypatch):
+    """Gradients, hooks, an overridden method, autocast, tables or rows of another type: the tensor operations run, and
+    give what they gave."""
+    from svoo_amd.processor import WanAttn_SAPAttn_Processor
+
+    say("heads: fallbacks")
+    heads, d, s = 2, 128, 40
+    layer = Layer(heads, d, heads * d, gpu)
+    x = torch.randn(1, s, heads * d, device=gpu, dtype=torch.bfloat16)
+    proc = _processor(WanAttn_SAPAttn_Processor)
+    cos, sin = (t[None, :, None] for t in _tables(s, d, gpu))
+    rope = dict(rotary_emb=(cos, sin))
+    assert _heads(proc, layer, x, False, monkeypatch, **rope)[1] == 1
+    # gradients: the weights' reach the result
+    for weight in (layer.norm_q.weight, layer.to_q.weight):
+        layer.requires_grad_(False)
+        weight.requires_grad_(True)
+        _, n = _heads(proc, layer, x, False, monkeypatch, **rope)
+        assert n == 0 and proc.got[0].requires_grad
+    with torch.no_grad():
+        assert _heads(proc, layer, x, False, monkeypatch, **rope)[1] == 1
+    layer.requires_grad_(False)
+    # a hook of the norm runs
+    seen = []
+    hook = layer.norm_k.register_forward_hook(lambda m, i, o: seen.append(1))
+    _heads(proc, layer, x, False, monkeypatch, **rope)
+    assert seen == [1]
+    hook.remove()
+    for kw, run in ((dict(rotary_emb=(cos.double(), sin.double())), x), (rope, x.expand(2, -1, -1).contiguous())):
+        want, n0 = _heads(proc, layer, run, True, monkeypatch, **kw)
+        got, n1 = _heads(proc, layer, run, False, monkeypatch, **kw)
+        assert n0 == n1 == 0 and all(torch.equal(a, b) for a, b in zip(got, want))
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert _heads(proc, layer, x, False, monkeypatch, **rope)[1] == 0
+    type(proc).get_qk_norm = lambda self, attn, q, k: (q, k)
+    assert _heads(proc, layer, x, False, monkeypatch, **rope)[1] == 0
