@@ -466,7 +466,11 @@ constexpr int kAsgTok = 4 * kAsgTokWave;
 // candidate pass could not settle.  Every block streams all of E, so a short list runs fastest on one column
 // block per wave (more blocks, each a quarter of the MFMA work): the candidate passes leave about 0.6% of the
 // keys at C3 from a warm start, one 512-token block per head with four column blocks (80-87 us per pass
-// against 38-41 us with one).  The certified pass's longer lists keep four.
+// against 38-41 us with one).  The certified pass leaves 7-15% of the keys: with at most kFbShortTokens tokens in all
+// that is fewer blocks of four column blocks than the chip has CUs, each a long serial chain, and one column block is
+// faster (per 5-iteration clustering, ten passes: 393 thousand tokens of 12 heads 320 us with four, 130 with one;
+// 786 thousand 449 and 208; 1.3 million 664 and 287; 2.0 million 315 and 211); above, four keep the E traffic down
+// (2.85 million, 24 heads: 596 and 657 us; 3.0 million, 40 heads: 409 and 411).
 template <bool LIST, int NCB>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 cocluster_assign_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ e_hi,
@@ -1713,8 +1717,8 @@ static int prep_launch(const uint16_t* a, const uint16_t* b, uint16_t* e_hi, uin
   return check_launch("svoo_cocluster_prep");
 }
 
-// short_list: the list is expected to hold a small share of the tokens (the candidate pass's leftovers): one
-// column block per wave.
+// short_list: the list is expected to be short (the candidate pass's leftovers, or the certified pass's of few
+// tokens): one column block per wave.
 static int assign_launch(const uint16_t* x, const uint16_t* e_hi, const uint16_t* e_lo, int32_t* labels, int bh, int n,
                          int j, int jpad, hipStream_t stream, int2* changes = nullptr, int32_t* nchanges = nullptr,
                          const int32_t* list = nullptr, const int32_t* list_count = nullptr, bool short_list = false) {
@@ -1729,6 +1733,8 @@ static int assign_launch(const uint16_t* x, const uint16_t* e_hi, const uint16_t
                        stream, x, e_hi, e_lo, labels, n, j, jpad, changes, nchanges, nullptr, nullptr);
   return check_launch("svoo_cocluster_assign");
 }
+
+static const long long kFbShortTokens = 1ll << 21;
 
 // The certified fp16 pass, then the hi + lo kernel on the tokens it left (fb_count must be zero on entry).
 // With bnd (and t_head) the pass records the pruning bounds; with list it runs on the listed tokens only.
@@ -1758,7 +1764,8 @@ static int assign16_launch(const uint16_t* x, const uint16_t* e16, const uint16_
                          nullptr);
   }
   if (int rc = check_launch("svoo_co_cluster (fp16 assign)")) return rc;
-  return assign_launch(x, e_hi, e_lo, labels, bh, n, j, jpad, stream, changes, nchanges, fb_list, fb_count);
+  return assign_launch(x, e_hi, e_lo, labels, bh, n, j, jpad, stream, changes, nchanges, fb_list, fb_count,
+                       (long long)bh * n <= kFbShortTokens);
 }
 
 static const int kMaxClusters = 4096;
