@@ -140,6 +140,17 @@ __global__ void zero_i32_kernel(int32_t* __restrict__ p, long long n) {
   if (i < n) p[i] = 0;
 }
 
+// Clears what a clustering needs at zero: two fp64 and two int32 ranges in one launch.
+__global__ void __launch_bounds__(256) zero_ranges_kernel(double* __restrict__ a, long long na, double* __restrict__ b,
+                                                          long long nb, int32_t* __restrict__ c, long long nc,
+                                                          int32_t* __restrict__ d, long long nd) {
+  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x, step = (long long)gridDim.x * blockDim.x;
+  for (long long i = t; i < na; i += step) a[i] = 0.0;
+  for (long long i = t; i < nb; i += step) b[i] = 0.0;
+  for (long long i = t; i < nc; i += step) c[i] = 0;
+  for (long long i = t; i < nd; i += step) d[i] = 0;
+}
+
 constexpr int kDeltaBlocks = 1024;  // waves split the change list (its length is on the device) into pieces
 constexpr int kDeltaBatch = 8;      // rows gathered at once per wave
 
@@ -229,6 +240,14 @@ int svoo_zero_i32(int32_t* p, long long n, hipStream_t stream) {
   if (n <= 0) return SVOO_OK;
   hipLaunchKernelGGL(zero_i32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, p, n);
   return check_launch("zero_i32");
+}
+
+int svoo_zero_ranges(double* a, long long na, double* b, long long nb, int32_t* c, long long nc, int32_t* d,
+                     long long nd, hipStream_t stream) {
+  const long long most = max(max(na, nb), max(nc, nd));
+  const unsigned blocks = (unsigned)min((most + 255) / 256, 4096ll);
+  hipLaunchKernelGGL(zero_ranges_kernel, dim3(blocks), dim3(256), 0, stream, a, na, b, nb, c, nc, d, nd);
+  return check_launch("zero_ranges");
 }
 
 // An incremental iteration's centroid update (the co-clustering's later passes): the move kernel (delta or

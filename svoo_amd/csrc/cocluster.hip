@@ -1681,7 +1681,8 @@ int svoo_centroid_move_impl(const uint16_t* x, const int32_t* sorted_idx, const 
                             uint16_t* new_c, int bh, int n, int k, int limit, hipStream_t stream, int32_t* zp,
                             long long zn);
 int svoo_zero_i32(int32_t* p, long long n, hipStream_t stream);
-int svoo_zero_f64(double* p, long long n, hipStream_t stream);
+int svoo_zero_ranges(double* a, long long na, double* b, long long nb, int32_t* c, long long nc, int32_t* d,
+                     long long nd, hipStream_t stream);
 
 static inline int pad_to(int v, int m) { return (v + m - 1) / m * m; }
 
@@ -1966,11 +1967,10 @@ extern "C" int svoo_co_cluster(const uint16_t* q, const uint16_t* k, int bh, int
   // changed tokens above which an iteration recounts every cluster instead of moving the changed ones
   const int limit = (int)((long long)bh * n / 32);
   const int jpad_k = pad_to(kc, kAssignChunk), jpad_q = pad_to(qc, kAssignChunk);
-  int rc = svoo_zero_f64(sums_k, (long long)bh * kc * 128, s);
-  if (!rc) rc = svoo_zero_f64(sums_q, (long long)bh * qc * 128, s);
-  if (!rc) rc = svoo_zero_i32(nch, 2 * kCounterStride, s);
-  // the per-pass counters start at zero; each side's finalize clears them again for the next side's prep
-  if (!rc) rc = svoo_zero_i32((int32_t*)stats, (long long)stats_words, s);
+  // the sums, the change counters and the per-pass counters start at zero (each side's finalize clears the last again
+  // for the next side's prep)
+  int rc = svoo_zero_ranges(sums_k, (long long)bh * kc * 128, sums_q, (long long)bh * qc * 128, nch,
+                            2 * kCounterStride, (int32_t*)stats, (long long)stats_words, s);
   // One side of an iteration: profiles of x's tokens live in the other side's centroid space.
   // A full iteration sorts the labels and sums every cluster (sums zero on entry, kept on exit); an
   // incremental one lists the tokens whose label changed and moves only their rows between the kept fp64

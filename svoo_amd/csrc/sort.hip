@@ -14,6 +14,12 @@
 //               4-byte writes merge in that XCD's L2 (81 -> 58 us per key-side sort at C3).
 // A launch of the three passes sorts the rows of one or two independent sorts (SortSide), so that the
 // co-clustering's two final sorts share their launches.
+// Short rows (at most kSortSmallN tokens and kSortSmallK clusters) take one kernel instead: one block per row, wave w
+// over the tokens [w, w + 1) / 16 of it in order, a histogram per wave in LDS, the scan over (cluster, wave) and the
+// ballot-ranked scatter.  Three launches of 4-8 us each were most of a short sort's time (and of one that its guard
+// switches off): 2 rows of 4680 tokens, 64 clusters 16.5 -> 8.7 us, 12 x 12288, 1000 clusters 26.6 -> 21.0; at 16384
+// tokens the two take the same (27.1 and 26.1 us, 20.9 and 21.3 with 100 clusters), as one CU's scattered stores set
+// the time of a row.
 #include "svoo_common.h"
 
 namespace svoo {
@@ -179,6 +185,101 @@ __global__ void __launch_bounds__(64) sort_scatter_kernel(SortSide sa, SortSide 
   }
 }
 
+constexpr int kSortSmallN = 12288;
+constexpr int kSortSmallK = 1024;
+constexpr int kSortSmallThreads = 1024;
+constexpr int kSortSmallWaves = kSortSmallThreads / kWave;
+
+// One block per row: the three passes in one launch (k <= kSortSmallK, n <= kSortSmallN; LDS int32 [16][k]).
+__global__ void __launch_bounds__(kSortSmallThreads) sort_small_kernel(SortSide sa, SortSide sb, int bh_a, int n,
+                                                                       int32_t* __restrict__ err,
+                                                                       const int32_t* __restrict__ guard, int limit,
+                                                                       double* __restrict__ zs, long long zn) {
+  if (guard && *guard <= limit) return;
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  if (zs)
+    for (long long i = (long long)blockIdx.x * kSortSmallThreads + tid; i < zn; i += (long long)gridDim.x * kSortSmallThreads)
+      zs[i] = 0.0;
+  extern __shared__ int32_t hist[];  // [wave][cluster]: counts, then the next position of that wave's tokens
+  __shared__ int wsum[kSortSmallWaves];
+  const bool second = (int)blockIdx.x >= bh_a;
+  const SortSide& S = second ? sb : sa;
+  const int b = second ? blockIdx.x - bh_a : blockIdx.x, k = S.k;
+  for (int i = tid; i < kSortSmallWaves * k; i += kSortSmallThreads) hist[i] = 0;
+  __syncthreads();
+  // the wave's tokens: `rounds` groups of 64, at most 16, all in registers
+  const int rounds = ((n + kWave - 1) / kWave + kSortSmallWaves - 1) / kSortSmallWaves;
+  const int t0 = wave * rounds * kWave;
+  const int32_t* lab = S.labels + (size_t)b * n;
+  int32_t* mine = hist + wave * k;
+  constexpr int kRounds = kSortSmallN / kSortSmallThreads;
+  int l[kRounds];
+  bool bad = false;
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    const int t = t0 + r * kWave + lane;
+    l[r] = r < rounds && t < n ? lab[t] : -1;
+  }
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    const int t = t0 + r * kWave + lane;
+    if ((unsigned)l[r] < (unsigned)k) {
+      atomicAdd(&mine[l[r]], 1);
+    } else {
+      bad |= r < rounds && t < n;
+      l[r] = -1;
+    }
+  }
+  if (bad && err) atomicOr(err, 1);
+  __syncthreads();
+  // thread i: cluster i over the waves (k <= 1024 threads)
+  int tot = 0;
+  if (tid < k) {
+#pragma unroll
+    for (int w = 0; w < kSortSmallWaves; ++w) tot += hist[w * k + tid];
+  }
+  const int inc = wave_inclusive_scan(tot, lane);
+  if (lane == kWave - 1) wsum[wave] = inc;
+  __syncthreads();
+  int before = 0;
+#pragma unroll
+  for (int w = 0; w < kSortSmallWaves; ++w) before += w < wave ? wsum[w] : 0;
+  if (tid < k) {
+    int run = before + inc - tot;
+    S.offsets[(size_t)b * k + tid] = run;
+    S.sizes[(size_t)b * k + tid] = tot;
+#pragma unroll
+    for (int w = 0; w < kSortSmallWaves; ++w) {
+      const int c = hist[w * k + tid];
+      hist[w * k + tid] = run;
+      run += c;
+    }
+  }
+  __syncthreads();
+  int32_t* out = S.sorted_idx + (size_t)b * n;
+  int32_t* outl = S.sorted_labels ? S.sorted_labels + (size_t)b * n : nullptr;
+  const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    if (r >= rounds) break;  // block-uniform
+    const int v = l[r];
+    unsigned long long same = __ballot(v >= 0);
+    for (int bit = 0; bit < S.kbits; ++bit) {
+      const bool on = (v >> bit) & 1;
+      const unsigned long long bal = __ballot(on);
+      same &= on ? bal : ~bal;
+    }
+    if (v >= 0) {
+      const int rank = __popcll(same & below), cnt = __popcll(same);
+      const int base = mine[v];
+      out[base + rank] = t0 + r * kWave + lane;
+      if (outl) outl[base + rank] = v;
+      if (rank == cnt - 1) mine[v] = base + cnt;
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
 }  // namespace svoo
 
 using namespace svoo;
@@ -206,6 +307,11 @@ static int sort_launch(const SortSide& sa, const SortSide& sb, int bh_a, int bh_
   const int nch = sort_nchunks(n), rows = bh_a + bh_b, kmax = max(sa.k, bh_b ? sb.k : 0);
   SVOO_REQUIRE((long long)kmax * nch < (1ll << 31), SVOO_ERR_UNSUPPORTED,
                "svoo_cluster_sort: k=%d x %d chunks too large", kmax, nch);
+  if (n <= kSortSmallN && kmax <= kSortSmallK) {
+    hipLaunchKernelGGL(sort_small_kernel, dim3(rows), dim3(kSortSmallThreads), kSortSmallWaves * kmax * sizeof(int32_t),
+                       stream, sa, sb, bh_a, n, err, guard, limit, zero_sums, zero_n);
+    return check_launch("svoo_cluster_sort");
+  }
   hipLaunchKernelGGL(sort_hist_kernel, dim3(nch, rows), dim3(256), kmax * sizeof(int32_t), stream, sa, sb, bh_a, n,
                      nch, err, guard, limit, zero_sums, zero_n);
   hipLaunchKernelGGL(sort_scan_kernel, dim3(rows), dim3(kScanWaves * kWave), 0, stream, sa, sb, bh_a, nch, guard,

@@ -77,6 +77,29 @@ def test_cluster_sort_bit_exact(gpu, bh, n, k):
     np.testing.assert_array_equal(slab.cpu().numpy(), np.take_along_axis(labels, oidx.astype(np.int64), 1))
 
 
+@pytest.mark.parametrize("bh,n,k", [(2, 12288, 1024), (3, 12289, 1024), (2, 12288, 1025), (5, 63, 3), (1, 1025, 7)])
+def test_cluster_sort_at_the_one_launch_rule(gpu, bh, n, k):
+    """Both sides of the rule that sorts short rows in one launch (at most 12288 tokens and 1024 clusters), rows shorter
+    than a wave, and labels outside the range, which are dropped: the rest is the stable order."""
+    from svoo_amd.permute import cluster_sort
+
+    say("cluster_sort, one-launch rule", bh, n, k)
+    r = np.random.default_rng(n * k)
+    labels = r.integers(0, k, size=(bh, n))
+    idx, sizes, offs, slab = cluster_sort(torch.from_numpy(labels).to(gpu), k, with_sorted_labels=True)
+    oidx, osz, ooff = O.cluster_sort(labels, k)
+    for got, want in ((idx, oidx), (sizes, osz), (offs, ooff), (slab, np.take_along_axis(labels, oidx.astype(np.int64), 1))):
+        np.testing.assert_array_equal(got.cpu().numpy(), want)
+    labels[:, ::5] = k
+    labels[:, 1::7] = -1
+    idx, sizes, offs = cluster_sort(torch.from_numpy(labels).to(gpu), k)
+    for b in range(bh):
+        ok = (labels[b] >= 0) & (labels[b] < k)
+        want = np.argsort(np.where(ok, labels[b], k), kind="stable")[: int(ok.sum())]
+        np.testing.assert_array_equal(idx[b].cpu().numpy()[: len(want)], want)
+        np.testing.assert_array_equal(sizes[b].cpu().numpy(), np.bincount(labels[b][ok], minlength=k))
+
+
 @pytest.mark.parametrize("d", [128, 32, 256])  # rows of 256 B (one step per block), 64 B, 512 B
 def test_permute_unpermute_bit_exact(gpu, d):
     from svoo_amd.permute import (apply_inverse_permutation, apply_inverse_permutation_bshd,
