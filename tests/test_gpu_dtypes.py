@@ -54,6 +54,30 @@ def test_convert_matches_torch_rounding(gpu):
     _same_bits(_lib.convert(v, torch.bfloat16), v.contiguous().to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("offset", [0, 1, 4])
+@pytest.mark.parametrize("src", [torch.bfloat16, torch.float16, torch.float32])
+def test_convert_vectors_tails_and_offsets(gpu, src, offset):
+    """Eight elements per lane, or one for buffers off 16-byte addresses and row widths that are no multiple of 8: lengths
+    around a vector, and rows padded and cut, against torch's casts."""
+    from svoo_amd import _lib
+
+    say("svoo_convert lengths and rows", src, offset)
+    base = torch.randn(70000, generator=torch.Generator().manual_seed(3)).to(src).to(gpu)
+    for dst in (torch.bfloat16, torch.float16, torch.float32):
+        for n in (1, 7, 8, 9, 17, 2049, 65537):
+            x = base[offset: offset + n]
+            if src != dst:
+                _same_bits(_lib.convert(x, dst), x.float().to(dst))
+        for rows, a, b in ((3, 64, 128), (33, 96, 128), (5, 63, 128), (17, 128, 40), (9, 128, 128), (7, 8, 24)):
+            x = base[offset: offset + rows * a].view(rows, a)
+            out = torch.full((rows, b), 7.0, dtype=dst, device=gpu)
+            _lib.call("svoo_convert_rows", x.data_ptr(), _lib._ELEM_TYPES[src], a, out.data_ptr(),
+                      _lib._ELEM_TYPES[dst], b, rows, _lib.stream_of(out.device))
+            want = torch.zeros(rows, b, dtype=dst, device=gpu)
+            want[:, : min(a, b)] = x[:, : min(a, b)].float().to(dst)
+            _same_bits(out, want)
+
+
 def _rand(shape, dtype, seed, gpu):
     g = torch.Generator().manual_seed(seed)
     return (torch.randn(shape, generator=g) * 1.7).to(dtype).to(gpu)
