@@ -162,7 +162,12 @@ __global__ void __launch_bounds__(256) cocluster_prep_kernel(const uint16_t* __r
 //   phase 2: row norms of praw (kept in LDS as bf16, which it is exactly), fp64;
 //   phase 3: E = inv * (praw B) on v_mfma_f32_32x32x16_bf16 (exact products, fp32 sums over the profile
 //            width; fp64 on the 16x16x4 MFMA cost as much as phase 1 again), with B staged through LDS in
-//            64-row chunks of 144-element rows, each requested from memory two chunks ahead.
+//            64-row chunks of 144-element rows, two buffers, each requested from memory two chunks ahead.
+// What bounds it: phase 1 at the fp64 MFMA's rate (one 16-column tile takes 1.75 us of a SIMD, measured with per-block
+// stamps; a second accumulator chain changes nothing), and on few blocks the fixed parts: the norms read LDS eight
+// values at a time (with one, 3.9 us at 1000 columns, now 2.3) and both halves of a wave share the epilogue, which one
+// half did alone (3.7 -> 2.5 us).  Per launch: 24 -> 18 us (key side) and 34 -> 25 (query side) at 12 heads, 500 and 100
+// clusters; 68 -> 62 and 67 -> 64 at 40 heads, 1000 and 100.
 constexpr int kPmRows = 16;
 constexpr int kPmChunk = 64;
 constexpr int kPmChunkStride = 144;
@@ -173,7 +178,7 @@ static inline __host__ __device__ size_t pm_praw_bytes(int kp) {
   return (size_t)kPmRows * (pm_kpp(kp) + 8) * sizeof(uint16_t);
 }
 static inline size_t pm_smem(int kp) {
-  return pm_praw_bytes(kp) + kPmRows * sizeof(double) + (size_t)kPmChunk * kPmChunkStride * sizeof(uint16_t);
+  return pm_praw_bytes(kp) + kPmRows * sizeof(double) + (size_t)2 * kPmChunk * kPmChunkStride * sizeof(uint16_t);
 }
 
 // Element offset of E16[row][col] within a head: 32-row tiles of 8 KB, each [k-step 0..7][lane 0..63][8],
@@ -201,12 +206,12 @@ __global__ void __launch_bounds__(256) cocluster_prep_mfma_kernel(const uint16_t
                                                                   int32_t* __restrict__ t_out, int have_old,
                                                                   uint16_t* __restrict__ praw_out,
                                                                   double* __restrict__ inv_out,
-                                                                  float* __restrict__ nrm_out) {
+                                                                  float* __restrict__ nrm_out, double sqrt_kp) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int kpp = pm_kpp(kp), ps = kpp + 8;
   uint16_t* praw = (uint16_t*)smem;                             // [16][ps] bf16
   double* inv = (double*)(smem + pm_praw_bytes(kp));           // [16]
-  uint16_t* bch = (uint16_t*)(inv + kPmRows);                   // [64][144] bf16
+  uint16_t* bch = (uint16_t*)(inv + kPmRows);                   // [2][64][144] bf16
   const int bidx = blockIdx.y, r0 = blockIdx.x * kPmRows;
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, li = lane % 16, q = lane / 16;
   const uint16_t* ab = a + (size_t)bidx * j * 128;
@@ -262,10 +267,17 @@ __global__ void __launch_bounds__(256) cocluster_prep_mfma_kernel(const uint16_t
   // Phase 2: inv = 1 / sqrt(sum + 1e-8), 16 threads per row.
   {
     const int r = tid / 16, sub = tid % 16;
+    // eight LDS reads in flight, summed in column order
     double sq = 0.0;
-    for (int k = sub; k < kp; k += 16) {
-      const double v = (double)bf16_to_f32(praw[r * ps + k]);
-      sq += v * v;
+    for (int k = sub; k < kp; k += 128) {
+      uint16_t p[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) p[i] = praw[r * ps + min(k + 16 * i, kpp - 1)];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const double v = k + 16 * i < kp ? (double)bf16_to_f32(p[i]) : 0.0;
+        sq += v * v;
+      }
     }
 #pragma unroll
     for (int o = 8; o > 0; o >>= 1) sq += __shfl_xor(sq, o);
@@ -307,9 +319,10 @@ __global__ void __launch_bounds__(256) cocluster_prep_mfma_kernel(const uint16_t
   const int toff = (8 * (grp / 2) + s16 / 4) * kPmChunkStride + dd0 + 16 * (grp % 2) + 4 * (s16 % 4);
   const int poff = (lane % 16) * ps + 8 * (lane / 32);
   uint32_t bmax = 0;  // max |B| as bf16 magnitude bits (they order like the values)
-  // Stage the chunk held in r (rows c ..), request chunk c + 2 * kPmChunk into r, then the chunk's MFMAs.
-  auto chunk_step = [&](u32x4_t(&r)[4], int c) {
-    __syncthreads();  // the previous chunk is consumed
+  // Stage the chunk held in r (rows c ..) into buffer bch, request chunk c + 2 * kPmChunk into r, then the chunk's MFMAs.
+  // The two buffers alternate, so one barrier per chunk: a buffer is written again after the barrier of the chunk
+  // between, which every wave reaches with its reads of it done.
+  auto chunk_step = [&](u32x4_t(&r)[4], int c, uint16_t* bch) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       *(u32x4_t*)(bch + (tid / 16 + 16 * i) * kPmChunkStride + (tid % 16) * 8) = r[i];
@@ -328,9 +341,19 @@ __global__ void __launch_bounds__(256) cocluster_prep_mfma_kernel(const uint16_t
       acc3 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(bt), as_bf16x8(pr), acc3, 0, 0, 0);
     }
   };
+  // the previous E's values for the change bounds, requested before the products
+  double old[2][4] = {};
+  if (e_old && have_old && r0 + lane % 16 < jpad) {
+    const double* eo = e_old + ((size_t)bidx * jpad + r0 + lane % 16) * 128 + dd0 + 4 * (lane / 32) + (lane & 16);
+#pragma unroll
+    for (int qi = 0; qi < 2; ++qi) {
+      const double2 o01 = *(const double2*)(eo + 8 * qi), o23 = *(const double2*)(eo + 8 * qi + 2);
+      old[qi][0] = o01.x, old[qi][1] = o01.y, old[qi][2] = o23.x, old[qi][3] = o23.y;
+    }
+  }
   for (int c = 0; c < kpp; c += 2 * kPmChunk) {
-    chunk_step(pre0, c);
-    if (c + kPmChunk < kpp) chunk_step(pre1, c + kPmChunk);
+    chunk_step(pre0, c, bch);
+    if (c + kPmChunk < kpp) chunk_step(pre1, c + kPmChunk, bch + kPmChunk * kPmChunkStride);
   }
   uint16_t* hb = e_hi + (size_t)bidx * jpad * 128;
   uint16_t* lb = e_lo + (size_t)bidx * jpad * 128;
@@ -348,25 +371,28 @@ __global__ void __launch_bounds__(256) cocluster_prep_mfma_kernel(const uint16_t
     __syncthreads();
     if (bmax) {
       int ex;
-      frexp(sqrt((double)kp) * (double)bf16_to_f32((uint16_t)bmax), &ex);  // bound < 2^ex
+      frexp(sqrt_kp * (double)bf16_to_f32((uint16_t)bmax), &ex);  // bound < 2^ex
       t_scale = 15 - ex;
     }
     if (t_out && tid == 0) t_out[bidx] = t_scale;  // the same value from every block of the head
   }
-  // Lane l with l % 32 < 16 holds row r = l % 16 at columns dd0 + 8 (v / 4) + 4 (l / 32) + v % 4 (v = 0..15).
+  // Lane l holds row r = l % 16 at columns dd0 + 8 (v / 4) + 4 (l / 32) + v % 4 (v = 0..15), lanes r and r + 16 the
+  // same values: the first takes v < 8, the second the rest.
   float err2 = 0.0f, nrm2 = 0.0f, dl2 = 0.0f;
   const int rr = lane % 16, row = r0 + rr;
+  const bool upper = (lane & 16) != 0;
   // Slots 4q .. 4q + 3 are four consecutive columns: each array gets one 8-byte store per group (the fp64 copy
   // two 16-byte accesses) instead of four 2-byte (8-byte) ones.
-  if ((lane % 32) < 16 && row < jpad) {
+  if (row < jpad) {
 #pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) {
-      const int dd = dd0 + 8 * q4 + 4 * (lane / 32);
+    for (int qi = 0; qi < 2; ++qi) {
+      const int dd = dd0 + 8 * (qi + (upper ? 2 : 0)) + 4 * (lane / 32);
       uint16_t hi[4], lo[4], h16b[4];
       double ev[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const double e = (double)acc3[4 * q4 + i] * inv[rr];
+        const float a3 = upper ? acc3[8 + 4 * qi + i] : acc3[4 * qi + i];
+        const double e = (double)a3 * inv[rr];
         ev[i] = e;
         hi[i] = f32_to_bf16((float)e);
         lo[i] = f32_to_bf16((float)(e - (double)bf16_to_f32(hi[i])));
@@ -376,12 +402,7 @@ __global__ void __launch_bounds__(256) cocluster_prep_mfma_kernel(const uint16_t
       *(uint2*)(lb + (size_t)row * 128 + dd) =
           make_uint2(lo[0] | ((uint32_t)lo[1] << 16), lo[2] | ((uint32_t)lo[3] << 16));
       if (e16) {
-        double old[4];
         double* eo = e_old ? e_old + ((size_t)bidx * jpad + row) * 128 + dd : nullptr;
-        if (eo && have_old) {
-          const double2 o01 = *(const double2*)eo, o23 = *(const double2*)(eo + 2);
-          old[0] = o01.x, old[1] = o01.y, old[2] = o23.x, old[3] = o23.y;
-        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           // padding rows (row >= j) are zero in the fp16 copy: their score is exactly 0
@@ -393,7 +414,7 @@ __global__ void __launch_bounds__(256) cocluster_prep_mfma_kernel(const uint16_t
           h16b[i] = __builtin_bit_cast(uint16_t, h16);
           if (eo && have_old) {
             // change of E since the previous call on this buffer (for the pruning bounds)
-            const double df = ev[i] - old[i];
+            const double df = ev[i] - old[qi][i];
             dl2 += (float)(df * df);
           }
         }
@@ -408,7 +429,10 @@ __global__ void __launch_bounds__(256) cocluster_prep_mfma_kernel(const uint16_t
   }
   if (e16) {
     // Per-row |2^t E_j - E16_j| and |E16_j| (rows of real clusters only), then the head's maxima.  A row's 128
-    // columns are spread over lanes r and r + 32 of each of the 4 waves.
+    // columns are spread over lanes r, r + 16, r + 32 and r + 48 of each of the 4 waves.
+    err2 += __shfl_xor(err2, 16);
+    nrm2 += __shfl_xor(nrm2, 16);
+    dl2 += __shfl_xor(dl2, 16);
     err2 += __shfl_xor(err2, 32);
     nrm2 += __shfl_xor(nrm2, 32);
     dl2 += __shfl_xor(dl2, 32);
@@ -1704,7 +1728,7 @@ static int prep_launch(const uint16_t* a, const uint16_t* b, uint16_t* e_hi, uin
   if (kp <= kPmMaxKp) {
     hipLaunchKernelGGL(cocluster_prep_mfma_kernel, dim3(jpad / kPmRows, bh), dim3(256), pm_smem(kp), stream, a, b,
                        e_hi, e_lo, profile, j, kp, jpad, e16, err_max, norm_max, e_old, delta, delta_max, t_out,
-                       have_old, praw_out, inv_out, nrm_out);
+                       have_old, praw_out, inv_out, nrm_out, sqrt((double)kp));
     return check_launch("svoo_cocluster_prep");
   }
   // Wide profiles: the vector kernel.  Few rows -> 2 rows per block for more blocks; many -> 8.

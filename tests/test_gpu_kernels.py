@@ -77,6 +77,25 @@ def test_cluster_sort_bit_exact(gpu, bh, n, k):
     np.testing.assert_array_equal(slab.cpu().numpy(), np.take_along_axis(labels, oidx.astype(np.int64), 1))
 
 
+@pytest.mark.parametrize("j,kp", [(1, 1), (17, 63), (64, 64), (33, 65), (5, 128), (20, 129), (16, 1407), (70, 1408), (9, 1409)])
+def test_profile_and_assignment_matrix_widths(gpu, j, kp):
+    """The prep at profile widths around its 64-row chunks (their two buffers alternate), with one chunk, and up to the
+    widest that the matrix kernel takes and one above: P against float64, E = P B within bf16 hi + lo (2^-16 of a term's
+    magnitude sum, the fp32 sums of kp products another kp 2^-24)."""
+    from svoo_amd.co_clustering import cocluster_profile
+
+    say("profile widths", j, kp)
+    a, at = rand_bf16((2, j, 128), j + kp, gpu)
+    b, bt = rand_bf16((2, kp, 128), j + kp + 1, gpu)
+    prof, e_hi, e_lo = cocluster_profile(at, bt)
+    want = O.profile_centroids(a, b)
+    np.testing.assert_allclose(prof.cpu().numpy(), want, rtol=1e-6, atol=1e-7)
+    e = (e_hi.double() + e_lo.double()).cpu().numpy()[:, :j]
+    p64, b64 = want.astype(np.float64), b.astype(np.float64)
+    size = np.abs(p64) @ np.abs(b64)
+    assert (np.abs(e - p64 @ b64) <= (2.0 ** -15 + kp * 2.0 ** -23) * size + 1e-12).all()
+
+
 @pytest.mark.parametrize("bh,n,k", [(2, 12288, 1024), (3, 12289, 1024), (2, 12288, 1025), (5, 63, 3), (1, 1025, 7)])
 def test_cluster_sort_at_the_one_launch_rule(gpu, bh, n, k):
     """Both sides of the rule that sorts short rows in one launch (at most 12288 tokens and 1024 clusters), rows shorter
