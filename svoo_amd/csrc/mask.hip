@@ -10,7 +10,8 @@
 //   that fail this test (2-3% of them on centroid data), or whose rows hold bf16 subnormals (which the MFMA
 //   may flush), are computed exactly in fp64: by their lane, or (for the mask) by the mask kernel.
 //
-// block_mask_kernel (one 256-thread block per (b, h, q-cluster) row):
+// block_mask_kernel (one 256-thread block per (b, h, q-cluster) row) and block_mask_wave_kernel (one wave per row, for
+// many rows of at most 1024 clusters):
 //   p_j  = bf16(f32(w_j e^(t_j - max) / max(sum, 1e-12)))   weighted softmax, evaluated in fp64
 //   order (p desc, j asc), found by two-level histograms of the bf16 bits of p (no sort)
 //   prefix_t = sum_{u<=t} floor(p_u * 2^60)  (exact int64) -> bf16 -> compared with bf16(top_p)
@@ -21,6 +22,7 @@
 namespace svoo {
 
 constexpr int kMaskThreads = 256;
+constexpr int kWaveRows = 2048;  // rows from which a wave each is faster than a block each (svoo_block_mask)
 
 constexpr int kScoreThreads = 256;
 
@@ -492,6 +494,235 @@ __global__ void __launch_bounds__(kMaskThreads) block_mask_kernel(uint16_t* __re
   if (tid == 0 && lengths) lengths[row] = len;
 }
 
+// The same row by one wave, E entries per lane (entry u * 64 + lane), without block barriers: a block of 256 threads per
+// row spent most of its time at some 17 of them and in wave 0's scans.  Differences from the block's kernel, none in a
+// result: the exponential comes from a table (within 1.3 units of the last place of float64, far below the rounding to
+// float32 and bf16) and the quotient from one reciprocal with a correction step, and a bin's count and mass share one
+// 32-bit LDS counter: a key of exponent e holds (128 + mantissa) 2^(e - 74) of the 2^60, so a bin's mass is a sum of
+// integers below 2^18 times a power of two (below e = 74 each entry is rounded down on its own, as the mass demands).
+// The score and size loads are issued together on clamped indexes (a guarded load waits for the one before it: 11.7k of
+// a row's 46k cycles, then 1.7k).  What is left is the exact dots of the deferred scores (a third of a row: 25 of 1000
+// entries) and the softmax.  Measured on 4000 rows of 1000: 33 us by blocks, 24.9 us by waves; eight gathered rows in
+// flight per group instead of four: 25.6 us (134 registers, fewer waves).
+template <int E>
+__global__ void __launch_bounds__(kMaskThreads) block_mask_wave_kernel(uint16_t* __restrict__ scores,
+                                                                       const uint16_t* __restrict__ qc,
+                                                                       const uint16_t* __restrict__ kc,
+                                                                       const int32_t* __restrict__ ksz,
+                                                                       const int32_t* __restrict__ preserve,
+                                                                       const int32_t* __restrict__ cap, int h, int qn,
+                                                                       int kn, long long rows, float inv_sqrt_d,
+                                                                       float p_st, uint8_t* __restrict__ map,
+                                                                       int32_t* __restrict__ lengths) {
+  constexpr int kW = kMaskThreads / kWave;
+  __shared__ double tab[64];
+  __shared__ uint32_t hist_s[kW][2][kBins];
+  __shared__ uint16_t dlist_s[kW][E * kWave], tfix_s[kW][E * kWave];
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  if (tid < 64) tab[tid] = kExp2Table[tid];
+  __syncthreads();
+  const long long row = (long long)blockIdx.x * kW + wave;
+  if (row >= rows) return;
+  const int bh = (int)(row / qn), head = bh % h;
+  uint32_t* h1 = hist_s[wave][0];
+  uint32_t* h2 = hist_s[wave][1];
+  uint16_t* dlist = dlist_s[wave];
+  uint16_t* tfix = tfix_s[wave];
+  uint8_t* mrow = map + row * kn;
+  uint16_t* trow = scores + row * kn;
+  const uint16_t* kb = kc + (size_t)bh * kn * 128;
+  const int32_t* wrow = ksz + (size_t)bh * kn;
+
+  // Scores, and the entries left to be computed exactly: 16 at a time, four per group of 16 lanes.
+  uint16_t tb[E];
+  int wt[E];
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
+    const int j = min(u * kWave + lane, kn - 1);  // (conditional loads would each wait for the one before)
+    tb[u] = trow[j];
+    wt[u] = wrow[j];
+  }
+  int nd = 0;
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
+    const int j = u * kWave + lane;
+    const bool def = j < kn && tb[u] == kDeferredScore;
+    const uint64_t b = __ballot(def);
+    if (def) dlist[nd + (int)__popcll(b & ((1ull << lane) - 1ull))] = (uint16_t)j;
+    nd += (int)__popcll(b);
+  }
+  if (nd > 0) {
+    const u32x4_t qw = ((const u32x4_t*)(qc + row * 128))[lane % 16];
+    constexpr int kR = 4;  // rows in flight per group
+    for (int base = 0; base < nd; base += 4 * kR) {
+      int jj[kR];
+      u32x4_t kw[kR];
+#pragma unroll
+      for (int t = 0; t < kR; ++t) {
+        const int slot = base + 4 * t + lane / 16;
+        jj[t] = slot < nd ? dlist[slot] : -1;
+        kw[t] = ((const u32x4_t*)(kb + (size_t)max(jj[t], 0) * 128))[lane % 16];
+      }
+#pragma unroll
+      for (int t = 0; t < kR; ++t) {
+        double acc = 0.0;  // the sum of group16_dot128
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          acc = fma((double)bf16_to_f32((uint16_t)(qw[e] & 0xffffu)), (double)bf16_to_f32((uint16_t)(kw[t][e] & 0xffffu)), acc);
+          acc = fma((double)bf16_to_f32((uint16_t)(qw[e] >> 16)), (double)bf16_to_f32((uint16_t)(kw[t][e] >> 16)), acc);
+        }
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
+        if (jj[t] >= 0 && lane % 16 == 0) {
+          const uint16_t bits = f32_to_bf16(bf16_to_f32(f32_to_bf16((float)acc)) * inv_sqrt_d);
+          tfix[jj[t]] = bits;
+          trow[jj[t]] = bits;
+        }
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int u = 0; u < E; ++u)
+      if (u * kWave + lane < kn && tb[u] == kDeferredScore) tb[u] = tfix[u * kWave + lane];
+  }
+  float m = -INFINITY;
+#pragma unroll
+  for (int u = 0; u < E; ++u) m = fmaxf(m, u * kWave + lane < kn ? bf16_to_f32(tb[u]) : -INFINITY);
+  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+
+  // Weighted softmax in fp64 -> bf16 probability keys.
+  double we[E];
+  double lsum = 0.0;
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
+    we[u] = 0.0;
+    if (u * kWave + lane < kn) {
+      we[u] = (double)wt[u] * exp_tab(tab, (double)bf16_to_f32(tb[u]) - (double)m);
+      lsum += we[u];
+    }
+  }
+  const double den = fmax(lane_f64(wave_scan_f64(lsum), kWave - 1), 1e-12);
+  const double rden = 1.0 / den;
+  uint32_t key[E];
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
+    const double q = we[u] * rden;
+    key[u] = f32_to_bf16((float)fma(fma(-q, den, we[u]), rden, q));
+  }
+
+  // Level 1: per exponent bin count << 20 | sum of (128 + mantissa).
+  h1[lane] = 0;
+  h1[lane + kWave] = 0;
+  h2[lane] = 0;
+  h2[lane + kWave] = 0;
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
+    if (u * kWave + lane < kn) {
+      const int e = (int)(key[u] >> 7);
+      uint32_t c = 128u + (key[u] & 127u);
+      if (e < 74) c = e > 66 ? c >> (74 - e) : 0u;
+      if (e >= 255) c = 0u;  // a NaN key, from NaN scores: no mass, in the top bin
+      atomicAdd(&h1[e & (kBins - 1)], (1u << 20) | c);
+    }
+  }
+  __builtin_amdgcn_wave_barrier();
+  // Lane l: positions 2l, 2l + 1 = bins 127 - 2l, 126 - 2l; the first bin whose prefix leaves the threshold.
+  const int b0 = kBins - 1 - 2 * lane, b1 = b0 - 1;
+  const uint32_t w0 = h1[b0], w1 = h1[b1];
+  const int c0 = (int)(w0 >> 20), c1 = (int)(w1 >> 20);
+  const long long m0 = (long long)(w0 & 0xfffffu) << max(b0 - 74, 0), m1 = (long long)(w1 & 0xfffffu) << max(b1 - 74, 0);
+  const int ci = wave_scan_i32(c0 + c1), ce = ci - c0 - c1;
+  const long long mi = wave_scan_i64(m0 + m1), me = mi - m0 - m1;
+  // Counts per mantissa of one bin (its values, one each) into h2.
+  auto level2 = [&](int bin) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < E; ++u)
+      if (u * kWave + lane < kn && (int)((key[u] >> 7) & (kBins - 1)) == bin) atomicAdd(&h2[key[u] & 127u], 1u);
+    __builtin_amdgcn_wave_barrier();
+  };
+  long long T = kn;  // leading positions whose prefix stays within the threshold
+  int dstar = -1;
+  {
+    const bool out0 = !prefix_within(me + m0, p_st), out1 = !prefix_within(mi, p_st);
+    const uint64_t any = __ballot(out0 || out1);
+    if (any != 0) {
+      const int l = __builtin_ctzll(any);
+      const bool first = (__ballot(out0) >> l) & 1;
+      dstar = first ? 2 * l : 2 * l + 1;
+      const long long base_m = lane_i64(first ? me : me + m0, l);
+      const int base_c = __builtin_amdgcn_readlane(first ? ce : ce + c0, l);
+      const int bstar = kBins - 1 - dstar;
+      level2(bstar);
+      const uint32_t k0 = ((uint32_t)bstar << 7) | (uint32_t)b0, k1 = ((uint32_t)bstar << 7) | (uint32_t)b1;
+      const int d0 = (int)h2[b0], d1 = (int)h2[b1];
+      const long long f0 = fixed60(k0), f1 = fixed60(k1);
+      const long long n0 = (long long)d0 * f0, n1 = (long long)d1 * f1;
+      const int di = wave_scan_i32(d0 + d1), de = di - d0 - d1;
+      const long long ni = wave_scan_i64(n0 + n1), ne = ni - n0 - n1;
+      const bool o0 = !prefix_within(base_m + ne + n0, p_st), o1 = !prefix_within(base_m + ni, p_st);
+      const uint64_t any2 = __ballot(o0 || o1);
+      const int l2 = __builtin_ctzll(any2 | (1ull << 63));
+      const bool f2 = (__ballot(o0) >> l2) & 1;
+      const long long mb = base_m + lane_i64(f2 ? ne : ne + n0, l2);
+      const long long fx = lane_i64(f2 ? f0 : f1, l2);
+      // smallest r in [0, cnt) with the prefix mb + (r + 1) fx outside the threshold
+      int lo = 0, hi = __builtin_amdgcn_readlane(f2 ? d0 : d1, l2) - 1;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (!prefix_within(mb + (long long)(mid + 1) * fx, p_st))
+          hi = mid;
+        else
+          lo = mid + 1;
+      }
+      T = base_c + __builtin_amdgcn_readlane(f2 ? de : de + d0, l2) + lo;
+    }
+  }
+  int len = 1 + (int)min(T, (long long)(kn - 1));
+  len = max(len, (int)preserve[head]);
+  if (cap[head] > 0) len = min(len, (int)cap[head]);
+  len = min(len, kn);
+
+  // The key and the rank among equal keys of position len - 1.
+  uint32_t key_l = 0;
+  int rank_l = 0;
+  if (len < kn) {
+    const bool r0 = ce + c0 >= len, r1 = ci >= len;
+    const int l = __builtin_ctzll(__ballot(r0 || r1));
+    const bool first = (__ballot(r0) >> l) & 1;
+    const int dl = first ? 2 * l : 2 * l + 1;
+    const int base_c = __builtin_amdgcn_readlane(first ? ce : ce + c0, l);
+    const int bl = kBins - 1 - dl;
+    if (dl != dstar) {
+      h2[lane] = 0;
+      h2[lane + kWave] = 0;
+      __builtin_amdgcn_wave_barrier();
+      level2(bl);
+    }
+    const int d0 = (int)h2[b0], d1 = (int)h2[b1];
+    const int di = wave_scan_i32(d0 + d1), de = di - d0 - d1;
+    const bool q0 = base_c + de + d0 >= len, q1 = base_c + di >= len;
+    const int l2 = __builtin_ctzll(__ballot(q0 || q1) | (1ull << 63));
+    const bool f2 = (__ballot(q0) >> l2) & 1;
+    key_l = ((uint32_t)bl << 7) | (uint32_t)(kBins - 1 - 2 * l2 - (f2 ? 0 : 1));
+    rank_l = len - 1 - (base_c + __builtin_amdgcn_readlane(f2 ? de : de + d0, l2));
+  }
+
+  // Kept: ahead of position len - 1 in (key desc, index asc).
+  int run = 0;
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
+    const int j = u * kWave + lane;
+    const uint64_t eq = __ballot(j < kn && key[u] == key_l);
+    const int rank = run + (int)__popcll(eq & ((1ull << lane) - 1ull));
+    run += (int)__popcll(eq);
+    const bool keep = len >= kn || key[u] > key_l || (key[u] == key_l && rank <= rank_l);
+    if (j < kn) mrow[j] = keep ? 1 : 0;
+  }
+  if (lane == 0 && lengths) lengths[row] = len;
+}
+
 // All-true map rows (top_p >= 1, svoo/co_clustering.py:575-576).
 __global__ void __launch_bounds__(kMaskThreads) full_mask_kernel(uint8_t* __restrict__ map, int qn, int kn,
                                                                  int32_t* __restrict__ lengths) {
@@ -578,10 +809,25 @@ extern "C" int svoo_block_mask(const uint16_t* qc, const uint16_t* kc, const int
 #define SVOO_MASK_LAUNCH(KP)                                                                                     \
   hipLaunchKernelGGL(block_mask_kernel<KP>, grid, dim3(kMaskThreads), 0, s, scores, qc, kc, k_sizes, preserve, cap, \
                      h, qn, kn, inv, p_storage, map, lengths)
+#define SVOO_MASK_WAVES(E)                                                                                       \
+  hipLaunchKernelGGL(block_mask_wave_kernel<E>, wgrid, dim3(kMaskThreads), 0, s, scores, qc, kc, k_sizes, preserve, cap, \
+                     h, qn, kn, rows, inv, p_storage, map, lengths)
+  // A row per wave or per block. A wave's row has no barriers and leaves room for many rows on a CU, a block's row is
+  // done sooner; the wave is ahead once there are some eight rows per CU, and always where a lane holds four entries.
+  // Block -> wave, Gaussian centroids, d 128: 200 clusters 6.4 -> 6.4 us at 200 rows, 43.6 -> 20.9 at 10240;
+  // 500 clusters 8.8 -> 9.5 at 600 rows, 11.0 -> 10.7 at 1200, 17.6 -> 12.9 at 2400, 55.4 -> 30.3 at 10240;
+  // 1000 clusters 14.9 -> 16.5 at 1200 rows, 24.4 -> 20.3 at 2400, 77.6 -> 49.4 at 10240.
+  const long long rows = (long long)b * h * qn;
+  const bool waves = rows >= kWaveRows;
+  const dim3 wgrid((unsigned)((rows + kMaskThreads / kWave - 1) / (kMaskThreads / kWave)));
   if (kn <= 256)
-    SVOO_MASK_LAUNCH(256);
+    SVOO_MASK_WAVES(4);
+  else if (kn <= 512 && waves)
+    SVOO_MASK_WAVES(8);
   else if (kn <= 512)
     SVOO_MASK_LAUNCH(512);
+  else if (kn <= 1024 && waves)
+    SVOO_MASK_WAVES(16);
   else if (kn <= 1024)
     SVOO_MASK_LAUNCH(1024);
   else if (kn <= 2048)
@@ -589,6 +835,7 @@ extern "C" int svoo_block_mask(const uint16_t* qc, const uint16_t* kc, const int
   else
     SVOO_MASK_LAUNCH(4096);
 #undef SVOO_MASK_LAUNCH
+#undef SVOO_MASK_WAVES
   return check_launch("svoo_block_mask");
 }
 

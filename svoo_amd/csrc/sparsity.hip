@@ -9,9 +9,9 @@
 // first counted into a histogram of the 65536 bit patterns (16-bit counts, 128 KB of LDS, one LDS atomic per score),
 // and everything after that works on the distinct values, in descending order of value:
 //   1. the non-empty groups of 64 patterns are listed (about 130 of 1024 for scores of one scale);
-//   2. per listed group the wave's 64 lanes weigh the 64 counts and sum them (fp64);
-//   3. one wave scans the group masses to the group where the mass from the top first reaches threshold * total,
-//      and the 64 values of that group to the crossing value, whose multiplicity is exact.
+//   2. 16 lanes per listed group weigh its 64 counts and sum them (fp64);
+//   3. every wave scans the masses of its 64 groups, the waves' totals find the group where the mass from the top first
+//      reaches threshold * total, and its wave the crossing value among the group's 64, whose multiplicity is exact.
 // All masses are fp64 sums of fp32 weights times counts, so the count does not depend on summation order beyond
 // 2^-53 of the mass.
 //
@@ -38,83 +38,11 @@ __device__ __forceinline__ uint32_t sp_raw(uint32_t o) { return o < 0x8000u ? 0x
 // First pattern of wave w's 64 groups (orders 4096 w ..).
 __device__ __forceinline__ int sp_base(int w) { return (int)sp_raw((uint32_t)w * 4096) & ~4095; }
 
-// 2^(i / 64), i = 0 .. 63, correctly rounded; the kernels keep a copy in LDS.
-__device__ const double kSpExp2[64] = {
-    0x1.0000000000000p+0, 0x1.02c9a3e778061p+0, 0x1.059b0d3158574p+0, 0x1.0874518759bc8p+0,
-    0x1.0b5586cf9890fp+0, 0x1.0e3ec32d3d1a2p+0, 0x1.11301d0125b51p+0, 0x1.1429aaea92de0p+0,
-    0x1.172b83c7d517bp+0, 0x1.1a35beb6fcb75p+0, 0x1.1d4873168b9aap+0, 0x1.2063b88628cd6p+0,
-    0x1.2387a6e756238p+0, 0x1.26b4565e27cddp+0, 0x1.29e9df51fdee1p+0, 0x1.2d285a6e4030bp+0,
-    0x1.306fe0a31b715p+0, 0x1.33c08b26416ffp+0, 0x1.371a7373aa9cbp+0, 0x1.3a7db34e59ff7p+0,
-    0x1.3dea64c123422p+0, 0x1.4160a21f72e2ap+0, 0x1.44e086061892dp+0, 0x1.486a2b5c13cd0p+0,
-    0x1.4bfdad5362a27p+0, 0x1.4f9b2769d2ca7p+0, 0x1.5342b569d4f82p+0, 0x1.56f4736b527dap+0,
-    0x1.5ab07dd485429p+0, 0x1.5e76f15ad2148p+0, 0x1.6247eb03a5585p+0, 0x1.6623882552225p+0,
-    0x1.6a09e667f3bcdp+0, 0x1.6dfb23c651a2fp+0, 0x1.71f75e8ec5f74p+0, 0x1.75feb564267c9p+0,
-    0x1.7a11473eb0187p+0, 0x1.7e2f336cf4e62p+0, 0x1.82589994cce13p+0, 0x1.868d99b4492edp+0,
-    0x1.8ace5422aa0dbp+0, 0x1.8f1ae99157736p+0, 0x1.93737b0cdc5e5p+0, 0x1.97d829fde4e50p+0,
-    0x1.9c49182a3f090p+0, 0x1.a0c667b5de565p+0, 0x1.a5503b23e255dp+0, 0x1.a9e6b5579fdbfp+0,
-    0x1.ae89f995ad3adp+0, 0x1.b33a2b84f15fbp+0, 0x1.b7f76f2fb5e47p+0, 0x1.bcc1e904bc1d2p+0,
-    0x1.c199bdd85529cp+0, 0x1.c67f12e57d14bp+0, 0x1.cb720dcef9069p+0, 0x1.d072d4a07897cp+0,
-    0x1.d5818dcfba487p+0, 0x1.da9e603db3285p+0, 0x1.dfc97337b9b5fp+0, 0x1.e502ee78b3ff6p+0,
-    0x1.ea4afa2a490dap+0, 0x1.efa1bee615a27p+0, 0x1.f50765b6e4540p+0, 0x1.fa7c1819e90d8p+0
-};
-// float(exp(double(s - m))): 2^(n / 64) from the table times a polynomial in |r| <= ln2 / 128 (its next term is below
-// 2^-54), within one unit of the last place of the float64 exponential.  The library's exp costs about three times
-// the instructions, and its constants, kept in registers over the loop, spilled.  s <= m, or NaN.
+// float(exp(double(s - m))).  The library's exp costs about three times the instructions of exp_tab, and its constants,
+// kept in registers over the loop, spilled.  s <= m, or NaN.
 __device__ __forceinline__ float sp_weight(const double* exp2_tab, uint32_t raw, float scale, float m) {
   const float s = __uint_as_float(raw << 16) * scale;
-  double x = (double)(s - m);
-  x = x < -200.0 ? -200.0 : x;  // 0 as a float well before; a NaN stays
-  const double nd = __builtin_rint(x * 0x1.71547652b82fep+6);
-  const int n = (int)nd;
-  double r = fma(nd, -0x1.62e42fefa39efp-7, x);
-  r = fma(nd, -0x1.abc9e3b39803fp-62, r);
-  double p = fma(r, 1.0 / 120.0, 1.0 / 24.0);
-  p = fma(p, r, 1.0 / 6.0);
-  p = fma(p, r, 0.5);
-  p = fma(p * r, r, r);
-  const double t = exp2_tab[n & 63];
-  const double y = fma(t, p, t);
-  return (float)__builtin_ldexp(y, n >> 6);
-}
-
-// Inclusive scan over the wave in the VALU (DPP row shifts and broadcasts; lanes without a source add 0).
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_add_f64(double v) {
-  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, ROWS, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, ROWS, 0xf, false);
-  return v + __builtin_bit_cast(double, ((unsigned long long)(uint32_t)hi << 32) | (uint32_t)lo);
-}
-template <int CTRL, int ROWS>
-__device__ __forceinline__ int dpp_add_i32(int v) {
-  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
-}
-// The same within each row of 16 lanes.
-__device__ __forceinline__ double row_scan_f64(double v) {
-  v = dpp_add_f64<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8
-  v = dpp_add_f64<0x112, 0xf>(v);
-  v = dpp_add_f64<0x114, 0xf>(v);
-  return dpp_add_f64<0x118, 0xf>(v);
-}
-__device__ __forceinline__ int row_scan_i32(int v) {
-  v = dpp_add_i32<0x111, 0xf>(v);
-  v = dpp_add_i32<0x112, 0xf>(v);
-  v = dpp_add_i32<0x114, 0xf>(v);
-  return dpp_add_i32<0x118, 0xf>(v);
-}
-__device__ __forceinline__ double wave_scan_f64(double v) {
-  v = dpp_add_f64<0x142, 0xa>(row_scan_f64(v));  // row_bcast:15 into rows 1 and 3
-  return dpp_add_f64<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
-}
-__device__ __forceinline__ int wave_scan_i32(int v) {
-  v = dpp_add_i32<0x142, 0xa>(row_scan_i32(v));
-  return dpp_add_i32<0x143, 0xc>(v);
-}
-__device__ __forceinline__ double lane_f64(double v, int lane) {
-  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
-  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+  return (float)exp_tab(exp2_tab, (double)(s - m));
 }
 
 // The wave's number, and a value that is the same in its lanes, in scalar registers.
@@ -128,7 +56,7 @@ struct SpShared {
   uint32_t hist[32768];                // pattern b: 16 bits at half b & 1 of word b >> 1
   double mass[kSpGroups];              // per group of orders: the mass of its scores
   int32_t cnt[kSpGroups];              // and their number
-  double exp2_tab[64];                 // kSpExp2
+  double exp2_tab[64];                 // kExp2Table
   double wmass[kSpWaves];              // the same per wave's 64 groups
   int32_t wcnt[kSpWaves];
   uint16_t list[kSpGroups];            // non-empty groups, from the top
@@ -300,7 +228,7 @@ __global__ void __launch_bounds__(kSpThreads) exact_count_kernel(const uint16_t*
   __shared__ __attribute__((aligned(16))) SpShared sh;
   const int tid = threadIdx.x, lane = tid % kWave;
   for (int i = tid; i < 32768 / 4; i += kSpThreads) ((u32x4_t*)sh.hist)[i] = u32x4_t{0u, 0u, 0u, 0u};
-  if (tid < 64) sh.exp2_tab[tid] = kSpExp2[tid];
+  if (tid < 64) sh.exp2_tab[tid] = kExp2Table[tid];
   u32x4_t v[NV];
   uint16_t edge = 0;
   auto load = [&](uint32_t row) {
@@ -349,7 +277,7 @@ __global__ void __launch_bounds__(kSpThreads) exact_count_long_kernel(const uint
   __shared__ __attribute__((aligned(16))) SpShared sh;
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
   for (int i = tid; i < 32768 / 4; i += kSpThreads) ((u32x4_t*)sh.hist)[i] = u32x4_t{0u, 0u, 0u, 0u};
-  if (tid < 64) sh.exp2_tab[tid] = kSpExp2[tid];
+  if (tid < 64) sh.exp2_tab[tid] = kExp2Table[tid];
   for (uint32_t row = blockIdx.x; row < rows; row += gridDim.x) {
     const SpRow r = sp_row(scores, row, n);
     const u32x4_t* src = (const u32x4_t*)(r.p + r.head);

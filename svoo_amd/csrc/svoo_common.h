@@ -114,6 +114,105 @@ __device__ __forceinline__ float xhalf_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// ---------------------------------------------------------------- float64 exponential from a table
+// 2^(i / 64), i = 0 .. 63, correctly rounded; kernels keep a copy in LDS.
+static __device__ const double kExp2Table[64] = {
+    0x1.0000000000000p+0, 0x1.02c9a3e778061p+0, 0x1.059b0d3158574p+0, 0x1.0874518759bc8p+0,
+    0x1.0b5586cf9890fp+0, 0x1.0e3ec32d3d1a2p+0, 0x1.11301d0125b51p+0, 0x1.1429aaea92de0p+0,
+    0x1.172b83c7d517bp+0, 0x1.1a35beb6fcb75p+0, 0x1.1d4873168b9aap+0, 0x1.2063b88628cd6p+0,
+    0x1.2387a6e756238p+0, 0x1.26b4565e27cddp+0, 0x1.29e9df51fdee1p+0, 0x1.2d285a6e4030bp+0,
+    0x1.306fe0a31b715p+0, 0x1.33c08b26416ffp+0, 0x1.371a7373aa9cbp+0, 0x1.3a7db34e59ff7p+0,
+    0x1.3dea64c123422p+0, 0x1.4160a21f72e2ap+0, 0x1.44e086061892dp+0, 0x1.486a2b5c13cd0p+0,
+    0x1.4bfdad5362a27p+0, 0x1.4f9b2769d2ca7p+0, 0x1.5342b569d4f82p+0, 0x1.56f4736b527dap+0,
+    0x1.5ab07dd485429p+0, 0x1.5e76f15ad2148p+0, 0x1.6247eb03a5585p+0, 0x1.6623882552225p+0,
+    0x1.6a09e667f3bcdp+0, 0x1.6dfb23c651a2fp+0, 0x1.71f75e8ec5f74p+0, 0x1.75feb564267c9p+0,
+    0x1.7a11473eb0187p+0, 0x1.7e2f336cf4e62p+0, 0x1.82589994cce13p+0, 0x1.868d99b4492edp+0,
+    0x1.8ace5422aa0dbp+0, 0x1.8f1ae99157736p+0, 0x1.93737b0cdc5e5p+0, 0x1.97d829fde4e50p+0,
+    0x1.9c49182a3f090p+0, 0x1.a0c667b5de565p+0, 0x1.a5503b23e255dp+0, 0x1.a9e6b5579fdbfp+0,
+    0x1.ae89f995ad3adp+0, 0x1.b33a2b84f15fbp+0, 0x1.b7f76f2fb5e47p+0, 0x1.bcc1e904bc1d2p+0,
+    0x1.c199bdd85529cp+0, 0x1.c67f12e57d14bp+0, 0x1.cb720dcef9069p+0, 0x1.d072d4a07897cp+0,
+    0x1.d5818dcfba487p+0, 0x1.da9e603db3285p+0, 0x1.dfc97337b9b5fp+0, 0x1.e502ee78b3ff6p+0,
+    0x1.ea4afa2a490dap+0, 0x1.efa1bee615a27p+0, 0x1.f50765b6e4540p+0, 0x1.fa7c1819e90d8p+0
+};
+// exp(x) for x <= 0 (or NaN): 2^(n / 64) from the table times a polynomial in |r| <= ln2 / 128 (its next term is below
+// 2^-54), within 1.3 units of the last place; x below -200 counts as -200 (its result is 0 in bf16 and fp32).
+__device__ __forceinline__ double exp_tab(const double* exp2_tab, double x) {
+  x = x < -200.0 ? -200.0 : x;  // a NaN stays
+  const double nd = __builtin_rint(x * 0x1.71547652b82fep+6);
+  const int n = (int)nd;
+  double r = fma(nd, -0x1.62e42fefa39efp-7, x);
+  r = fma(nd, -0x1.abc9e3b39803fp-62, r);
+  double p = fma(r, 1.0 / 120.0, 1.0 / 24.0);
+  p = fma(p, r, 1.0 / 6.0);
+  p = fma(p, r, 0.5);
+  p = fma(p * r, r, r);
+  const double t = exp2_tab[n & 63];
+  return __builtin_ldexp(fma(t, p, t), n >> 6);
+}
+
+// ---------------------------------------------------------------- wave scans and sums
+// Inclusive scan over the wave in the VALU (DPP row shifts and broadcasts; lanes without a source add 0).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add_f64(double v) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, ROWS, 0xf, false);
+  return v + __builtin_bit_cast(double, ((unsigned long long)(uint32_t)hi << 32) | (uint32_t)lo);
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_add_i32(int v) {
+  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
+// The same within each row of 16 lanes.
+__device__ __forceinline__ double row_scan_f64(double v) {
+  v = dpp_add_f64<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8
+  v = dpp_add_f64<0x112, 0xf>(v);
+  v = dpp_add_f64<0x114, 0xf>(v);
+  return dpp_add_f64<0x118, 0xf>(v);
+}
+__device__ __forceinline__ int row_scan_i32(int v) {
+  v = dpp_add_i32<0x111, 0xf>(v);
+  v = dpp_add_i32<0x112, 0xf>(v);
+  v = dpp_add_i32<0x114, 0xf>(v);
+  return dpp_add_i32<0x118, 0xf>(v);
+}
+__device__ __forceinline__ double wave_scan_f64(double v) {
+  v = dpp_add_f64<0x142, 0xa>(row_scan_f64(v));  // row_bcast:15 into rows 1 and 3
+  return dpp_add_f64<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+}
+__device__ __forceinline__ int wave_scan_i32(int v) {
+  v = dpp_add_i32<0x142, 0xa>(row_scan_i32(v));
+  return dpp_add_i32<0x143, 0xc>(v);
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ long long dpp_add_i64(long long v) {
+  const unsigned long long u = (unsigned long long)v;
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, ROWS, 0xf, false);
+  return v + (long long)(((unsigned long long)(uint32_t)hi << 32) | (uint32_t)lo);
+}
+__device__ __forceinline__ long long wave_scan_i64(long long v) {
+  v = dpp_add_i64<0x111, 0xf>(v);
+  v = dpp_add_i64<0x112, 0xf>(v);
+  v = dpp_add_i64<0x114, 0xf>(v);
+  v = dpp_add_i64<0x118, 0xf>(v);
+  v = dpp_add_i64<0x142, 0xa>(v);
+  return dpp_add_i64<0x143, 0xc>(v);
+}
+// A lane's value in every lane (the lane uniform).
+__device__ __forceinline__ long long lane_i64(long long v, int lane) {
+  const unsigned long long u = (unsigned long long)v;
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
+  return (long long)(((unsigned long long)hi << 32) | lo);
+}
+__device__ __forceinline__ double lane_f64(double v, int lane) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
 // ---------------------------------------------------------------- block reductions
 template <int kThreads>
 __device__ __forceinline__ double block_sum_f64(double v, double* scratch) {

@@ -274,6 +274,48 @@ def test_block_mask_bit_exact(gpu, p, mn, mx, qn, kn):
     np.testing.assert_array_equal(lens.cpu().numpy(), olens)
 
 
+@pytest.mark.parametrize(
+    "qn,kn",
+    [(5, 1), (5, 63), (5, 64), (5, 65), (5, 256), (5, 257), (409, 257), (411, 257), (411, 512), (5, 513), (411, 513)]
+    + [(411, 1001), (409, 1023), (411, 1023), (411, 1024), (411, 1025)],
+)
+def test_block_mask_row_widths(gpu, qn, kn):
+    """A row per wave (64 entries a step: up to 256 clusters, and up to 1024 from 2048 rows on) or per block, at the
+    widths and row counts around the rule (5 * 409 and 5 * 411 rows): Gaussian centroids, equal scores (ties in index
+    order), one dominant cluster with probabilities far below 2^-60 behind it, and sizes that are mostly zero; for
+    each the oracle's map and lengths."""
+    from svoo_amd.co_clustering import block_mask_lengths
+
+    say("block_mask widths", qn, kn)
+    (qc, kc, qs, ks), _ = _mask_case(gpu, 5, qn, kn, 7 * kn)
+    kc[0, 1] = kc[0, 1, :1]
+    kc[0, 2] *= 12.0
+    ks[0, 3, : kn - kn // 8] = 0
+    args = bf16(qc, gpu), bf16(kc, gpu), torch.from_numpy(qs).to(gpu), torch.from_numpy(ks).to(gpu)
+    for p, mn, mx in ((0.9, 0.1, 0), (0.0, [0.0, 0.3, 0.5, 0.9, 1.0], 0), (0.9999, 0, 0.5)):
+        m, lens = block_mask_lengths(*args, p, mn, mx)
+        om, olens = O.identify_dynamic_map(qc, O.bf16_round(kc), qs, ks, p, mn, mx, return_lengths=True)
+        np.testing.assert_array_equal(lens.cpu().numpy(), olens)
+        np.testing.assert_array_equal(m.cpu().numpy(), om)
+
+
+@pytest.mark.parametrize("kn", [257, 1000])
+def test_block_mask_infinite_scores_by_wave_and_block(gpu, kn):
+    """Scores of -inf (one cluster, half of them, all but one): 2050 rows (a wave each) give what the same rows give 1000 at a time (a block each)."""
+    from svoo_amd.co_clustering import block_mask_lengths
+
+    say("block_mask infinite", kn)
+    (qc, kc, qs, ks), _ = _mask_case(gpu, 5, 410, kn, kn)
+    qc = np.abs(qc) + np.float32(0.125)
+    kc[0, 1, 3], kc[0, 2, ::2], kc[0, 3, 1:, 7] = -np.inf, -np.inf, -np.inf
+    args = bf16(qc, gpu), bf16(kc, gpu), torch.from_numpy(qs).to(gpu), torch.from_numpy(ks).to(gpu)
+    m, lens = block_mask_lengths(*args, 0.9, 0.1, 0)
+    for i in (0, 205):
+        part = args[0][:, :, i : i + 200].contiguous(), args[1], args[2][:, :, i : i + 200].contiguous(), args[3]
+        mp, lp = block_mask_lengths(*part, 0.9, 0.1, 0)
+        assert torch.equal(m[:, :, i : i + 200], mp) and torch.equal(lens[:, :, i : i + 200], lp)
+
+
 def _score_cases():
     """(name, qc, kc) float32 arrays of bf16 values [1, H, n, 128] for the centroid-score kernel."""
     r = np.random.default_rng(77)
