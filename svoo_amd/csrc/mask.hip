@@ -47,87 +47,88 @@ __device__ __forceinline__ double group16_dot128(const uint16_t* __restrict__ x,
   return acc;
 }
 
-// 1 when any of the 8 bf16 values of w is subnormal (exponent 0, mantissa not 0).
-__device__ __forceinline__ uint32_t has_subnormal(u32x4_t w) {
-  uint32_t any = 0;
+// Folds 8 bf16 values, signs cleared, into a running minimum of (bits - 1): one of them was subnormal (exponent 0,
+// mantissa not 0) when a half ends below 0x7f.
+typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void fold_subnormal(u16x2_t& lowest, u32x4_t mag) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const uint32_t lo = w[e] & 0xffffu, hi = w[e] >> 16;
-    any |= ((lo & 0x7f80u) == 0 && (lo & 0x7fu) != 0) | ((hi & 0x7f80u) == 0 && (hi & 0x7fu) != 0);
-  }
-  return any;
+  for (int e = 0; e < 4; ++e)
+    lowest = __builtin_elementwise_min(lowest, (u16x2_t)(__builtin_bit_cast(u16x2_t, mag[e]) - (u16x2_t){1, 1}));
 }
+__device__ __forceinline__ bool found_subnormal(u16x2_t lowest) { return lowest.x < 0x7f || lowest.y < 0x7f; }
 
 // Marks an entry whose certificate failed when the exact dot is left to the mask kernel (not a value
 // f32_to_bf16 produces: its NaNs are 0x7fc0).
 constexpr uint16_t kDeferredScore = 0xffffu;
-// k-steps (16 products each) summed in fp32 per partial; the partials are added in fp64.  The certificate's
-// half-width is 2^-24 * 32 * kStepsPerPartial * a: twice the worst-case fp32 rounding of a partial of
-// 16 * kStepsPerPartial products, which also covers the fp32 error of a itself and the final rounding.
-constexpr int kStepsPerPartial = 1;
+// The certificate's half-width is kHalfWidth a: twice the worst-case fp32 rounding of a partial of one k-step (16
+// products; the partials are added in fp64), which also covers the fp32 error of a itself and the final rounding.
+constexpr float kHalfWidth = 0x1p-24f * 32.0f;
 
 // Lane layout (v_mfma_f32_32x32x16_bf16, keys on M, query centroids on N): lane (l32, h) supplies key
-// row kt*32 + l32 and query row qt*32 + l32, the 8 values at d = 64h + 8s in k-step s (the same
-// permutation of the contraction index in both operands), and receives entry r at key (r/4)*8 + 4h + r%4,
-// query l32.  defer != 0 writes kDeferredScore for the entries that fail the certificate instead of
+// row kt*32 + l32 and query row qt*32 + l32, the 8 values at d = 16s + 8h in k-step s, and receives entry r at key (r/4)*8 + 4h + r%4,
+// query l32.  DEFER writes kDeferredScore for the entries that fail the certificate instead of
 // recomputing them.
-__global__ void __launch_bounds__(kScoreThreads) __attribute__((amdgpu_waves_per_eu(2, 8)))
+// Bound by the VALU (a tile is 256 float64 operations per lane, the certificate of 16 entries and the subnormal test
+// beside 16 MFMAs), so the test is three packed 16-bit operations per two values and the rounding the conversion
+// instruction.  The key tile is staged and tested once per block; registers for four waves per SIMD.  40 heads x 100
+// queries x 1000 keys: 26.6 us with 12 operations a word and 240 registers (two waves), 14.5 us now; 12 x 100 x 500:
+// 9.4 -> 6.2 us.  Five waves per SIMD spill (17.9 us).
+template <bool DEFER>
+__global__ void __launch_bounds__(kScoreThreads, DEFER ? 4 : 3)
 centroid_scores_kernel(const uint16_t* __restrict__ qc, const uint16_t* __restrict__ kc, int qn, int kn,
-                       float inv_sqrt_d, int defer, uint16_t* __restrict__ out) {
+                       float inv_sqrt_d, uint16_t* __restrict__ out) {
   const int b = blockIdx.y, kt = blockIdx.x;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, h = lane / 32, l32 = lane % 32;
   const int qtiles = (qn + 31) / 32;
-  const int jrow = min(kt * 32 + l32, kn - 1);
   const uint16_t* kbase = kc + (size_t)b * kn * 128;
   const uint16_t* qbase = qc + (size_t)b * qn * 128;
-  u32x4_t ka[8];
-  uint32_t ksub = 0;
-  {
-    const u32x4_t* src = (const u32x4_t*)(kbase + (size_t)jrow * 128) + 8 * h;
-#pragma unroll
-    for (int st = 0; st < 8; ++st) {
-      ka[st] = src[st];
-      ksub |= has_subnormal(ka[st]);
-    }
-  }
-  // key rows (of this tile) holding a subnormal, as a bit mask over l32
-  const uint64_t kmask64 = __ballot(ksub != 0);
-  const uint32_t kmask = (uint32_t)kmask64 | (uint32_t)(kmask64 >> 32);
   const u32x4_t absm = {0x7fff7fffu, 0x7fff7fffu, 0x7fff7fffu, 0x7fff7fffu};
-  const float half_width = 0x1p-24f * (float)(32 * kStepsPerPartial);
-  __shared__ uint16_t redo_list[kScoreThreads / kWave][kWave * 16];
+  // the key tile in LDS, 16-byte chunk c of row l at l * 16 + (c ^ l % 16); its rows holding a subnormal as bits
+  __shared__ u32x4_t ktile[32 * 16];
+  __shared__ uint32_t kmask_s;
+  if (threadIdx.x == 0) kmask_s = 0;
+  __syncthreads();
+#pragma unroll
+  for (int c = threadIdx.x; c < 32 * 16; c += kScoreThreads) {
+    const int l = c / 16;
+    const u32x4_t w = ((const u32x4_t*)(kbase + (size_t)min(kt * 32 + l, kn - 1) * 128))[c % 16];
+    u16x2_t kmin = {0xffff, 0xffff};
+    fold_subnormal(kmin, w & absm);
+    if (found_subnormal(kmin)) atomicOr(&kmask_s, 1u << l);
+    ktile[l * 16 + ((c ^ l) % 16)] = w;
+  }
+  __syncthreads();
+  const uint32_t kmask = kmask_s;
   for (int qt = wave; qt < qtiles; qt += kScoreThreads / kWave) {
     const int i = qt * 32 + l32, irow = min(i, qn - 1);
     u32x4_t qb[8];
-    uint32_t qsub = 0;
     {
-      const u32x4_t* src = (const u32x4_t*)(qbase + (size_t)irow * 128) + 8 * h;
+      const u32x4_t* src = (const u32x4_t*)(qbase + (size_t)irow * 128) + h;
 #pragma unroll
-      for (int st = 0; st < 8; ++st) {
-        qb[st] = src[st];
-        qsub |= has_subnormal(qb[st]);
+      for (int st = 0; st < 8; ++st) qb[st] = src[2 * st];
+    }
+    asm volatile("" ::: "memory");  // (the key tile is read again for each query tile, not kept in registers)
+    // partials of one k-step each, summed in fp64 as they come
+    u16x2_t qmin = {0xffff, 0xffff};
+    double sd[16];
+    f32x16_t asum = f32x16_t{};
+#pragma unroll
+    for (int st = 0; st < 8; ++st) {
+      const u32x4_t ka = ktile[l32 * 16 + ((2 * st + h) ^ (l32 % 16))];
+      const f32x16_t part = mfma32x32x16(as_bf16x8(ka), as_bf16x8(qb[st]), f32x16_t{});
+      const u32x4_t qm = qb[st] & absm;
+      asum = mfma32x32x16(as_bf16x8(ka & absm), as_bf16x8(qm), asum);
+      fold_subnormal(qmin, qm);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        sd[r] = st == 0 ? (double)part[r] : sd[r] + (double)part[r];
+        asm volatile("" : "+v"(sd[r]));  // (the sums are formed here: deferred to their use, all partials stay live)
       }
     }
     // this lane's query row holds a subnormal (either half)
+    const uint32_t qsub = found_subnormal(qmin) ? 1u : 0u;
     const auto qsw = __builtin_amdgcn_permlane32_swap(qsub, qsub, false, false);
-    const uint32_t qsub_row = qsw[0] | qsw[1];
-    // partials of kStepsPerPartial k-steps each, summed in fp64 as they come
-    double sd[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) sd[r] = 0.0;
-#pragma unroll
-    for (int p0 = 0; p0 < 8; p0 += kStepsPerPartial) {
-      f32x16_t part = f32x16_t{};
-#pragma unroll
-      for (int st = p0; st < p0 + kStepsPerPartial; ++st)
-        part = mfma32x32x16(as_bf16x8(ka[st]), as_bf16x8(qb[st]), part);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) sd[r] += (double)part[r];
-    }
-    f32x16_t asum = f32x16_t{};
-#pragma unroll
-    for (int st = 0; st < 8; ++st)
-      asum = mfma32x32x16(as_bf16x8(ka[st] & absm), as_bf16x8(qb[st] & absm), asum);
+    const uint32_t subs = (qsw[0] | qsw[1]) != 0 ? 0xffffffffu : kmask >> (4 * h);
     // entries whose certificate fails: bit r of `redo`
     uint32_t redo = 0;
 #pragma unroll
@@ -139,13 +140,13 @@ centroid_scores_kernel(const uint16_t* __restrict__ qc, const uint16_t* __restri
         const int r = 4 * g + e;
         const float rs = (float)sd[r];
         const float a = asum[r];
-        const float err = fmaf(a, half_width, 0x1p-118f);
-        const uint16_t sb = f32_to_bf16(rs - err);
-        const bool sub = ((kmask >> (g * 8 + 4 * h + e)) & 1u) != 0 || qsub_row != 0;
-        uint32_t tb = f32_to_bf16(bf16_to_f32(sb) * inv_sqrt_d);
-        if (sub || !(a <= 3.0e38f) || sb != f32_to_bf16(rs + err)) {
+        const float err = fmaf(a, kHalfWidth, 0x1p-118f);
+        const uint32_t both = cvt_pk_bf16(rs - err, rs + err);  // (a NaN comes with a > 3e38)
+        const bool sub = ((subs >> (g * 8 + e)) & 1u) != 0;
+        uint32_t tb = cvt_pk_bf16(__uint_as_float(both << 16) * inv_sqrt_d, 0.0f) & 0xffffu;
+        if (sub || !(a <= 3.0e38f) || (both & 0xffffu) != both >> 16) {
           redo |= 1u << r;
-          if (defer) tb = kDeferredScore;
+          if (DEFER) tb = kDeferredScore;
         }
         packed[e / 2] |= tb << (16 * (e % 2));
       }
@@ -161,7 +162,7 @@ centroid_scores_kernel(const uint16_t* __restrict__ qc, const uint16_t* __restri
     }
     // The failed entries again, exactly in fp64, four at a time by groups of 16 lanes (listed in this wave's
     // LDS slice as lane << 4 | r); their stores come after the first ones, in the same wave.
-    if (!defer) {
+    if constexpr (!DEFER) {
       if (i >= qn) redo = 0;
       const int nmine = __builtin_popcount(redo);
       int pos = nmine;
@@ -172,6 +173,7 @@ centroid_scores_kernel(const uint16_t* __restrict__ qc, const uint16_t* __restri
       }
       const int total = __shfl(pos, kWave - 1);
       pos -= nmine;
+      __shared__ uint16_t redo_list[kScoreThreads / kWave][kWave * 16];
       uint16_t* list = redo_list[wave];
       while (redo) {
         const int r = __builtin_ctz(redo);
@@ -780,8 +782,8 @@ extern "C" int svoo_centroid_scores(const uint16_t* qc, const uint16_t* kc, int 
   SVOO_REQUIRE_HEAD_DIM(d, "svoo_centroid_scores");
   SVOO_REQUIRE(bh <= 65535 && kn <= (1 << 26), SVOO_ERR_UNSUPPORTED, "svoo_centroid_scores: grid too large");
   const float inv = 1.0f / (float)sqrt((double)d);
-  hipLaunchKernelGGL(centroid_scores_kernel, dim3((kn + 31) / 32, bh), dim3(kScoreThreads), 0, (hipStream_t)stream,
-                     qc, kc, qn, kn, inv, 0, scores);
+  hipLaunchKernelGGL(centroid_scores_kernel<false>, dim3((kn + 31) / 32, bh), dim3(kScoreThreads), 0, (hipStream_t)stream,
+                     qc, kc, qn, kn, inv, scores);
   return check_launch("svoo_centroid_scores");
 }
 
@@ -803,8 +805,8 @@ extern "C" int svoo_block_mask(const uint16_t* qc, const uint16_t* kc, const int
   }
   const float inv = 1.0f / (float)sqrt((double)d);
   // scores with the uncertified entries deferred to the mask kernel, which computes them exactly
-  hipLaunchKernelGGL(centroid_scores_kernel, dim3((kn + 31) / 32, b * h), dim3(kScoreThreads), 0, s, qc, kc, qn, kn,
-                     inv, 1, scores);
+  hipLaunchKernelGGL(centroid_scores_kernel<true>, dim3((kn + 31) / 32, b * h), dim3(kScoreThreads), 0, s, qc, kc, qn, kn,
+                     inv, scores);
   if (int rc = check_launch("svoo_block_mask (scores)")) return rc;
 #define SVOO_MASK_LAUNCH(KP)                                                                                     \
   hipLaunchKernelGGL(block_mask_kernel<KP>, grid, dim3(kMaskThreads), 0, s, scores, qc, kc, k_sizes, preserve, cap, \

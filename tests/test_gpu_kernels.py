@@ -357,6 +357,26 @@ def test_centroid_scores_bit_exact(gpu, case):
     assert torch.equal(centroid_logits(bf16(qc, gpu), bf16(kc, gpu)), got)  # EAR's logits are the same values
 
 
+@pytest.mark.parametrize("qn,kn", [(1, 1), (31, 33), (32, 32), (33, 31), (129, 34), (160, 68)])
+def test_centroid_scores_tile_edges(gpu, qn, kn):
+    """Whole and partial tiles of 32 x 32, more query tiles than waves, and a subnormal value at the first, a middle
+    and the last place of a first and a last row: the exact scores, and the mask built on the deferred ones."""
+    from svoo_amd.co_clustering import block_mask_lengths, centroid_scores
+
+    say("centroid scores tiles", qn, kn)
+    (qc, kc, qs, ks), _ = _mask_case(gpu, 6, qn, kn, qn + kn)
+    for head, place in enumerate((0, 63, 127)):
+        qc[0, head, -1, place] = kc[0, head + 3, 0, place] = O.bf16_round(np.float32(2e-39)).item()
+        kc[0, head, -1, place] = qc[0, head + 3, 0, place] = O.bf16_round(np.float32(-1e-38)).item()
+    args = bf16(qc, gpu), bf16(kc, gpu)
+    got, want = centroid_scores(*args), O.centroid_scores(qc, kc)
+    np.testing.assert_array_equal(O.bf16_bits(f32(got)), O.bf16_bits(want))
+    m, lens = block_mask_lengths(*args, torch.from_numpy(qs).to(gpu), torch.from_numpy(ks).to(gpu), 0.9, 0.1, 0)
+    om, olens = O.identify_dynamic_map(qc, kc, qs, ks, 0.9, 0.1, 0, return_lengths=True)
+    np.testing.assert_array_equal(lens.cpu().numpy(), olens)
+    np.testing.assert_array_equal(m.cpu().numpy(), om)
+
+
 def _attn_check(out, ref):
     o = f32(out).astype(np.float64).reshape(-1)
     r = np.asarray(ref, np.float64).reshape(-1)
