@@ -677,8 +677,8 @@ class Hunyuan_SAPAttn_Processor(WanAttn_SAPAttn_Processor):
             return None
         if not double:
             return heads.qkv_heads(query, key, value, h, **norm, **kw)
-        # the text's keys are normed where its queries are (get_encoder_condition_and_concat)
-        text_norm = norm_args(("norm_added_q", "norm_added_k")) if getattr(attn, "norm_added_q", None) is not None else {}
+        # (the text's queries and keys are each normed where they have a norm; the pass takes both norms or none)
+        text_norm = norm_args(("norm_added_q", "norm_added_k"))
         if text_norm is None or text <= 0:
             return None
         projections = [getattr(attn, n, None) for n in ("add_q_proj", "add_k_proj", "add_v_proj")]

@@ -126,6 +126,30 @@ def test_hunyuan_heads_equal_the_operations(gpu, monkeypatch, heads, d, s, text,
         assert torch.equal(got[2], want[2])
 
 
+@pytest.mark.parametrize("q_norm,k_norm", [(True, False), (False, True), (False, False)])
+def test_hunyuan_text_norms_one_by_one(gpu, monkeypatch, q_norm, k_norm):
+    """A double-stream block with a norm for the text's queries only, its keys only or neither: each is normed where it
+    has a norm, whichever path runs."""
+    from svoo_amd.processor import Hunyuan_SAPAttn_Processor
+
+    say("hunyuan text norms", q_norm, k_norm)
+    torch.manual_seed(5)
+    heads, d, s, text = 3, 128, 40, 9
+    layer = Layer(heads, d, d, gpu, double=True)
+    if not q_norm:
+        layer.norm_added_q = None
+    if not k_norm:
+        layer.norm_added_k = None
+    x = torch.randn(1, s, heads * d, device=gpu, dtype=torch.bfloat16) * 3
+    txt = torch.randn(1, text, heads * d, device=gpu, dtype=torch.bfloat16) * 3
+    kw = dict(encoder_hidden_states=txt, image_rotary_emb=_tables(s, d, gpu))
+    proc = _processor(Hunyuan_SAPAttn_Processor)
+    want, _ = _heads(proc, layer, x, True, monkeypatch, **kw)
+    got, _ = _heads(proc, layer, x, False, monkeypatch, **kw)
+    _close(got[:2], want[:2])
+    assert torch.equal(got[2], want[2])
+
+
 def test_the_operations_run_where_the_pass_cannot(gpu, monkeypatch):
     """Gradients, hooks, an overridden method, autocast, tables or rows of another type: the tensor operations run, and
     give what they gave."""
