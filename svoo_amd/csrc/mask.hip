@@ -203,6 +203,8 @@ centroid_scores_kernel(const uint16_t* __restrict__ qc, const uint16_t* __restri
 // ------------------------------------------------------------------------------------------ block mask
 // The sort keys are the bf16 bits of p (p >= 0, so they order as unsigned integers like the values):
 // bin = key >> 7 (the exponent), sub-bin = key & 127 (the mantissa), so a sub-bin holds one value.
+// A NaN or +inf score, or only -inf ones, makes the row's sum NaN: there is no order then, and every key is 0, so that
+// the row keeps its first clusters up to the cap, all without one (the reference's comparisons with NaN remove nothing).
 constexpr int kBins = 128;
 
 // bf16(f32(x * 2^-60)) <= p_st for a fixed-point prefix x (monotone in x)
@@ -215,6 +217,11 @@ __device__ __forceinline__ long long fixed60(uint32_t key) {
   const float p = bf16_to_f32((uint16_t)key);
   return p > 0.0f ? (long long)ldexp((double)p, 60) : 0ll;
 }
+
+// The softmax's divisor: at least 1e-12; infinite for a NaN sum, which makes every key 0.
+__device__ __forceinline__ double softmax_divisor(double sum) { return sum != sum ? INFINITY : fmax(sum, 1e-12); }
+// The key of a probability (0 for a NaN).
+__device__ __forceinline__ uint32_t probability_key(double p) { return f32_to_bf16(fmaxf((float)p, 0.0f)); }
 
 // Inclusive scans over the 64 lanes of a wave.
 __device__ __forceinline__ long long wave_incl_scan_i64(long long v) {
@@ -330,10 +337,10 @@ __global__ void __launch_bounds__(kMaskThreads) block_mask_kernel(uint16_t* __re
       lsum += we[u];
     }
   }
-  const double den = fmax(block_sum_f64<kMaskThreads>(lsum, red_d), 1e-12);
+  const double den = softmax_divisor(block_sum_f64<kMaskThreads>(lsum, red_d));
   uint32_t key[E];
 #pragma unroll
-  for (int u = 0; u < E; ++u) key[u] = f32_to_bf16((float)(we[u] / den));
+  for (int u = 0; u < E; ++u) key[u] = probability_key(we[u] / den);
 
   // Level 1: counts and masses per exponent bin.
   if (tid < kBins) {
@@ -344,7 +351,6 @@ __global__ void __launch_bounds__(kMaskThreads) block_mask_kernel(uint16_t* __re
 #pragma unroll
   for (int u = 0; u < E; ++u) {
     if (tid * E + u < kn) {
-      // (a NaN key, from NaN scores, lands in the top bin instead of outside the table)
       atomicAdd(&cnt1[(key[u] >> 7) & (kBins - 1)], 1u);
       atomicAdd(&mass1[(key[u] >> 7) & (kBins - 1)], (unsigned long long)fixed60(key[u]));
     }
@@ -604,13 +610,13 @@ __global__ void __launch_bounds__(kMaskThreads) block_mask_wave_kernel(uint16_t*
       lsum += we[u];
     }
   }
-  const double den = fmax(lane_f64(wave_scan_f64(lsum), kWave - 1), 1e-12);
+  const double den = softmax_divisor(lane_f64(wave_scan_f64(lsum), kWave - 1));
   const double rden = 1.0 / den;
   uint32_t key[E];
 #pragma unroll
   for (int u = 0; u < E; ++u) {
     const double q = we[u] * rden;
-    key[u] = f32_to_bf16((float)fma(fma(-q, den, we[u]), rden, q));
+    key[u] = probability_key(fma(fma(-q, den, we[u]), rden, q));
   }
 
   // Level 1: per exponent bin count << 20 | sum of (128 + mantissa).
@@ -625,7 +631,6 @@ __global__ void __launch_bounds__(kMaskThreads) block_mask_wave_kernel(uint16_t*
       const int e = (int)(key[u] >> 7);
       uint32_t c = 128u + (key[u] & 127u);
       if (e < 74) c = e > 66 ? c >> (74 - e) : 0u;
-      if (e >= 255) c = 0u;  // a NaN key, from NaN scores: no mass, in the top bin
       atomicAdd(&h1[e & (kBins - 1)], (1u << 20) | c);
     }
   }

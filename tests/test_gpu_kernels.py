@@ -316,6 +316,43 @@ def test_block_mask_infinite_scores_by_wave_and_block(gpu, kn):
         assert torch.equal(m[:, :, i : i + 200], mp) and torch.equal(lens[:, :, i : i + 200], lp)
 
 
+@pytest.mark.parametrize("cap", [0, 0.3])
+@pytest.mark.parametrize("kn", [70, 257, 1000, 1500])
+def test_block_mask_rows_without_an_order(gpu, kn, cap):
+    """A row with a NaN or +inf score, or only -inf ones, has a NaN softmax sum and no order: it keeps its first
+    clusters up to the cap, all without one (as in the reference, where no comparison with NaN removes a cluster),
+    from the kernel of a wave per row and of a block per row alike; the other rows are as before."""
+    from svoo_amd.co_clustering import block_mask_lengths
+
+    say("block_mask without an order", kn, cap)
+    (qc, kc, qs, ks), _ = _mask_case(gpu, 5, 410, kn, kn)
+    clean = [bf16(qc, gpu), bf16(kc, gpu), torch.from_numpy(qs).to(gpu), torch.from_numpy(ks).to(gpu)]
+    want, wlen = block_mask_lengths(*clean, 0.9, 0.1, cap)
+    qc = qc.copy()
+    qc[0, 0, 3], qc[0, 2, 400], qc[0, 3, 0, 7] = np.nan, -np.inf, np.inf  # (all NaN, all NaN, +inf and -inf)
+    qc[0, 1, 5, 7], qc[0, 1, 6, 7] = np.inf, -np.inf  # all +inf, all -inf
+    kc = kc.copy()
+    kc[0, 1, :, 7] = np.abs(kc[0, 1, :, 7]) + np.float32(0.125)
+    kc[0, 4, 11] = np.nan  # one NaN score in every row of the head
+    rows = [(0, 3), (1, 5), (1, 6), (2, 400), (3, 0)] + [(4, i) for i in range(410)]
+    bad = torch.zeros(5, 410, dtype=torch.bool)
+    for h, i in rows:
+        bad[h, i] = True
+    args = bf16(qc, gpu), bf16(kc, gpu), clean[2], clean[3]
+    m, lens = block_mask_lengths(*args, 0.9, 0.1, cap)
+    keep = max(1, int(cap * kn)) if cap else kn
+    got = m[0].cpu()[bad]
+    assert (lens[0].cpu()[bad] == keep).all(), "lengths"
+    assert bool(got[:, :keep].all()) and not bool(got[:, keep:].any()), "kept clusters"
+    for h in (0, 2, 3):  # (head 1 has other key centroids)
+        ok = (~bad[h]).to(gpu)
+        assert torch.equal(m[0, h][ok], want[0, h][ok]) and torch.equal(lens[0, h][ok], wlen[0, h][ok])
+    for i in (0, 205):
+        part = args[0][:, :, i : i + 205].contiguous(), args[1], args[2][:, :, i : i + 205].contiguous(), args[3]
+        mp, lp = block_mask_lengths(*part, 0.9, 0.1, cap)
+        assert torch.equal(m[:, :, i : i + 205], mp) and torch.equal(lens[:, :, i : i + 205], lp)
+
+
 def _score_cases():
     """(name, qc, kc) float32 arrays of bf16 values [1, H, n, 128] for the centroid-score kernel."""
     r = np.random.default_rng(77)
