@@ -20,7 +20,7 @@
 // in registers while the current one is counted and scanned, so memory and LDS work overlap.  Measured on 12288 rows of
 // 32760 scores (805 MB): 9.28 ms with a fp64 exp and a wave-combined LDS update per score (three passes, 256 threads),
 // 0.34 ms here (2.3 TB/s); a row costs about 17 thousand cycles, 9 thousand of them independent of its length (9608
-// rows of 2402 scores: 0.56 -> 0.16 ms).
+// rows of 2402 scores: 0.56 -> 0.16 ms).  Many short rows take exact_count_short_kernel (the rule of short_rows).
 #include "svoo_common.h"
 
 namespace svoo {
@@ -343,9 +343,190 @@ __global__ void __launch_bounds__(kSpThreads) exact_count_long_kernel(const uint
   }
 }
 
+// ---------------------------------------------------------------- short rows
+// One block of 256 threads per row, several per CU, without the table of all patterns: the largest score; a 256-bin
+// histogram over the high byte of the key (counts and masses), whose scan finds the bin where the mass from the top
+// reaches threshold * total; counts over the low byte inside that bin, each sub-bin one exact value.
+constexpr int kShortThreads = 256;
+
+// Bit pattern -> key whose unsigned order is the numeric order.
+__device__ __forceinline__ uint32_t short_key(uint16_t b) { return 0xffffu - sp_order(b); }
+
+__device__ __forceinline__ float short_weight(uint32_t raw, float scale, float m) {
+  const float s = __uint_as_float(raw << 16) * scale;
+  return (float)exp((double)(s - m));
+}
+
+// Lanes of a wave with the same bin combine their (count, weight) before one LDS atomic per
+// distinct bin: scores concentrate in a few binades, and plain per-lane atomics would serialise.
+__device__ __forceinline__ double wave_sum_f64(double v) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  return v;
+}
+__device__ __forceinline__ void hist_add(int32_t* cnt, double* mass, int bin, double w, bool valid) {
+  const int lane = threadIdx.x & (kWave - 1);
+  unsigned long long todo = __ballot(valid);
+  while (todo) {
+    const int leader = __ffsll((long long)todo) - 1;
+    const int lb = __shfl(bin, leader);
+    const bool mine = valid && bin == lb;
+    const unsigned long long mm = __ballot(mine);
+    const double sum = wave_sum_f64(mine ? w : 0.0);
+    if (lane == leader) {
+      atomicAdd(&cnt[lb], (int)__popcll(mm));
+      atomicAdd(&mass[lb], sum);
+    }
+    todo &= ~mm;
+  }
+}
+__device__ __forceinline__ void count_add(int32_t* cnt, int bin, bool valid) {
+  const int lane = threadIdx.x & (kWave - 1);
+  unsigned long long todo = __ballot(valid);
+  while (todo) {
+    const int leader = __ffsll((long long)todo) - 1;
+    const int lb = __shfl(bin, leader);
+    const unsigned long long mm = __ballot(valid && bin == lb);
+    if (lane == leader) atomicAdd(&cnt[lb], (int)__popcll(mm));
+    todo &= ~mm;
+  }
+}
+
+// Inclusive prefix, from the top bin down, of the 256 bins' masses and counts (thread t holds bin
+// 255 - t); a fixed summation order.
+__device__ void short_scan(const int32_t* cnt, const double* mass, double* dsc, long long* isc) {
+  const int tid = threadIdx.x;
+  dsc[tid] = mass[255 - tid];
+  isc[tid] = cnt[255 - tid];
+  __syncthreads();
+  for (int off = 1; off < kShortThreads; off <<= 1) {
+    const double dv = tid >= off ? dsc[tid - off] : 0.0;
+    const long long iv = tid >= off ? isc[tid - off] : 0;
+    __syncthreads();
+    dsc[tid] += dv;
+    isc[tid] += iv;
+    __syncthreads();
+  }
+}
+
+// The bin (scanned from the top) at which the scanned mass first reaches `target`, with the mass
+// and count strictly above it; the lowest non-empty bin when rounding leaves the total below the
+// target.  Call after sp_scan.
+struct ShortCross {
+  int bin;
+  double mass_above;
+  long long cnt_above;
+};
+__device__ ShortCross short_find(const int32_t* cnt, double target, const double* dsc, const long long* isc, int* found) {
+  const int tid = threadIdx.x;
+  if (tid == 0) *found = -1;
+  __syncthreads();
+  const double above = tid > 0 ? dsc[tid - 1] : 0.0;
+  if (cnt[255 - tid] > 0 && above < target && dsc[tid] >= target) *found = tid;
+  __syncthreads();
+  if (*found < 0) {
+    __syncthreads();
+    if (tid == 0) {
+      int last = 0;
+      for (int i = 0; i < kShortThreads; ++i)
+        if (cnt[255 - i] > 0) last = i;
+      *found = last;
+    }
+    __syncthreads();
+  }
+  const int t = *found;
+  ShortCross r;
+  r.bin = 255 - t;
+  r.mass_above = t > 0 ? dsc[t - 1] : 0.0;
+  r.cnt_above = t > 0 ? isc[t - 1] : 0;
+  __syncthreads();
+  return r;
+}
+
+__global__ void __launch_bounds__(kShortThreads) exact_count_short_kernel(const uint16_t* __restrict__ scores, int n,
+                                                                   float scale, float threshold,
+                                                                   int32_t* __restrict__ counts) {
+  __shared__ int32_t cnt[256];
+  __shared__ double mass[256];
+  __shared__ double dsc[kShortThreads];
+  __shared__ long long isc[kShortThreads];
+  __shared__ int found;
+  __shared__ uint32_t kmax_s;
+  const size_t row = blockIdx.x;
+  const int tid = threadIdx.x;
+  const uint16_t* sr = scores + row * (size_t)n;
+
+  // 1. row max as a key
+  uint32_t kmax = 0;
+  for (int j = tid; j < n; j += kShortThreads) kmax = max(kmax, short_key(sr[j]));
+  for (int o = 32; o > 0; o >>= 1) kmax = max(kmax, (uint32_t)__shfl_xor((int)kmax, o));
+  if (tid == 0) kmax_s = 0;
+  cnt[tid] = 0;
+  mass[tid] = 0.0;
+  __syncthreads();
+  if ((tid & (kWave - 1)) == 0) atomicMax(&kmax_s, kmax);
+  __syncthreads();
+  const float m = bf16_to_f32((uint16_t)sp_raw(0xffffu - kmax_s)) * scale;
+
+  // 2. high-byte histogram of counts and weights (whole-wave iterations: every lane takes part)
+  for (int j0 = 0; j0 < n; j0 += kShortThreads) {
+    const int j = j0 + tid;
+    const bool valid = j < n;
+    const uint16_t b = valid ? sr[j] : (uint16_t)0;
+    const uint32_t k = short_key(b);
+    hist_add(cnt, mass, (int)(k >> 8), valid ? (double)short_weight(b, scale, m) : 0.0, valid);
+  }
+  __syncthreads();
+  short_scan(cnt, mass, dsc, isc);
+  const double total = dsc[kShortThreads - 1];
+  const double target = (double)threshold * total;
+  const ShortCross c1 = short_find(cnt, target, dsc, isc, &found);
+
+  // 3. low-byte counts inside the crossing bin; each sub-bin is one exact value
+  cnt[tid] = 0;
+  __syncthreads();
+  for (int j0 = 0; j0 < n; j0 += kShortThreads) {
+    const int j = j0 + tid;
+    const uint32_t k = j < n ? short_key(sr[j]) : 0u;
+    count_add(cnt, (int)(k & 255), j < n && (int)(k >> 8) == c1.bin);
+  }
+  __syncthreads();
+  {
+    const int sb = 255 - tid;
+    mass[sb] = (double)cnt[sb] * (double)short_weight(sp_raw(0xffffu - (((uint32_t)c1.bin << 8) | (uint32_t)sb)), scale, m);
+  }
+  __syncthreads();
+  short_scan(cnt, mass, dsc, isc);
+  const double rem = target - c1.mass_above;
+  const ShortCross c2 = short_find(cnt, rem, dsc, isc, &found);
+  if (tid == 0) {
+    const double v = (double)short_weight(sp_raw(0xffffu - (((uint32_t)c1.bin << 8) | (uint32_t)c2.bin)), scale, m);
+    const int mult = cnt[c2.bin];
+    const double need = rem - c2.mass_above;
+    long long k = 1;
+    if (v > 0.0 && need > 0.0) {
+      k = (long long)ceil(need / v);
+      // the smallest k with k * v >= need (the division may round either way)
+      while (k > 1 && (double)(k - 1) * v >= need) --k;
+      while (k < mult && (double)k * v < need) ++k;
+    }
+    k = k < 1 ? 1 : (k > mult ? mult : k);
+    counts[row] = (int32_t)(c1.cnt_above + c2.cnt_above + k);
+  }
+}
+
 }  // namespace svoo
 
 using namespace svoo;
+
+// Short rows go to the kernel of several small blocks per CU once there are rows enough: the histogram's rows cost one
+// CU about 3.7 us each whatever their length, in rounds of 256 rows, the small blocks' 9-15 us in all plus a share that
+// grows with the length.  Histogram -> small blocks: 64 scores 6.3 -> 10.5 us at 256 rows, 13.3 -> 10.8 at 513, 178 ->
+// 75 at 12288; 257 scores 10.5 -> 12.2 at 500, 17.7 -> 15.2 at 769; 385 scores 18.7 -> 20.8 at 1024, 36.7 -> 34.8 at
+// 2049; 513 scores 193 -> 186 at 12288; 600 scores 194 -> 216 at 12288, and always behind from there on.
+static bool short_rows(long long rows, int n) {
+  if (n > 544) return false;
+  return rows > 256 * (n <= 32 ? 1 : n <= 256 ? 2 : n <= 288 ? 3 : n <= 448 ? 8 : n <= 512 ? 16 : 32);
+}
 
 extern "C" int svoo_exact_sparsity_counts(const uint16_t* scores, long long rows, int n, float scale, float threshold,
                                           int32_t* counts, void* stream) {
@@ -354,9 +535,14 @@ extern "C" int svoo_exact_sparsity_counts(const uint16_t* scores, long long rows
                "svoo_exact_sparsity_counts: bad dims rows=%lld n=%d", rows, n);
   SVOO_REQUIRE(threshold > 0.0f && threshold <= 1.0f, SVOO_ERR_INVALID_ARG,
                "svoo_exact_sparsity_counts: threshold %g outside (0, 1]", (double)threshold);
+  hipStream_t s = (hipStream_t)stream;
+  if (short_rows(rows, n)) {
+    hipLaunchKernelGGL(exact_count_short_kernel, dim3((unsigned)rows), dim3(kShortThreads), 0, s, scores, n, scale,
+                       threshold, counts);
+    return check_launch("svoo_exact_sparsity_counts");
+  }
   // One block per CU (256 on MI355X): the histogram fills the LDS, and the rows are dealt round robin.
   const dim3 grid((unsigned)(rows < 256 ? rows : 256)), block(kSpThreads);
-  hipStream_t s = (hipStream_t)stream;
 #define SVOO_COUNT(K) hipLaunchKernelGGL(K, grid, block, 0, s, scores, (uint32_t)rows, n, scale, threshold, counts)
   if (n > kSpSingle) SVOO_COUNT(exact_count_long_kernel);
   else if (n <= 8 * kSpThreads) SVOO_COUNT(exact_count_kernel<1>);

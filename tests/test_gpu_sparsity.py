@@ -75,6 +75,27 @@ def test_counts_at_the_row_length_rules(gpu, n, kind):
         assert np.array_equal(got, O.exact_sparsity_counts(sc, 0.0884, thr)), (n, kind, thr)
 
 
+@pytest.mark.parametrize("rows,n", [(257, 1), (256, 32), (257, 32), (512, 33), (513, 33), (513, 256), (769, 257),
+                                    (769, 288), (2049, 289), (2049, 448), (4097, 449), (4097, 512), (8193, 513),
+                                    (8193, 544), (8193, 545)])
+def test_counts_of_many_short_rows(gpu, rows, n):
+    """Row counts and lengths on both sides of the rule between the kernel of many small blocks and the histogram's: the
+    oracle's counts, and those of the same rows 100 at a time (the histogram), -inf, +inf and NaN rows among them."""
+    from svoo_amd.sparsity import exact_counts_from_scores
+
+    say("exact counts of short rows", rows, n)
+    rng = np.random.default_rng(rows + n)
+    kinds = ("normal", "ties", "peaked", "equal")
+    sc = np.concatenate([_scores(rng, (rows + 3) // 4, n, k) for k in kinds])[:rows]
+    t = torch.from_numpy(sc).to(torch.bfloat16).to(gpu)
+    for thr in (0.5, 0.95):
+        assert np.array_equal(exact_counts_from_scores(t, 0.0884, thr).cpu().numpy(),
+                              O.exact_sparsity_counts(sc, 0.0884, thr)), (rows, n, thr)
+    t[0, n // 2:], t[1], t[2, n - 1], t[3, 0] = -np.inf, -np.inf, np.inf, np.nan
+    some = torch.cat([exact_counts_from_scores(t[i : i + 100], 0.0884, 0.95) for i in range(0, min(rows, 600), 100)])
+    assert torch.equal(exact_counts_from_scores(t, 0.0884, 0.95)[: some.numel()], some)
+
+
 def test_counts_of_masked_and_infinite_scores(gpu):
     """-inf (masked) scores weigh nothing; a row with +inf or NaN has no finite mass and counts every score above its
     lowest value, plus one."""
