@@ -485,31 +485,19 @@ __global__ void __launch_bounds__(256) cocluster_prep_mfma_kernel(const uint16_t
 constexpr int kAsgTokWave = 128;
 constexpr int kAsgTok = 4 * kAsgTokWave;
 
-// With LIST the block's tokens are entries [T x, T x + T) of the head's token list (T = 128 NCB; list[bidx][.],
-// count[bidx] entries; blocks past the count exit at once): the tokens the certified fp16 pass or the
-// candidate pass could not settle.  Every block streams all of E, so a short list runs fastest on one column
-// block per wave (more blocks, each a quarter of the MFMA work): the candidate passes leave about 0.6% of the
-// keys at C3 from a warm start, one 512-token block per head with four column blocks (80-87 us per pass
-// against 38-41 us with one).  The certified pass leaves 7-15% of the keys: with at most kFbShortTokens tokens in all
-// that is fewer blocks of four column blocks than the chip has CUs, each a long serial chain, and one column block is
-// faster (per 5-iteration clustering, ten passes: 393 thousand tokens of 12 heads 320 us with four, 130 with one;
-// 786 thousand 449 and 208; 1.3 million 664 and 287; 2.0 million 315 and 211); above, four keep the E traffic down
-// (2.85 million, 24 heads: 596 and 657 us; 3.0 million, 40 heads: 409 and 411).
+// Tokens [t0, t0 + 128 NCB) of a head: of all n tokens, or with LIST entries of the head's token list lst (ntok entries).
+// s_e: LDS [buffer][hi, lo].
+typedef uint16_t AssignLds[2][2][kAssignChunk * 128];
 template <bool LIST, int NCB>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-cocluster_assign_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ e_hi,
-                        const uint16_t* __restrict__ e_lo, int32_t* __restrict__ labels, int n, int j, int jpad,
-                        int2* __restrict__ changes, int32_t* __restrict__ nchanges,
-                        const int32_t* __restrict__ list, const int32_t* __restrict__ list_count) {
-  __shared__ __attribute__((aligned(16))) uint16_t s_e[2][2][kAssignChunk * 128];  // [buffer][hi, lo]
+__device__ __forceinline__ void assign_block(AssignLds& s_e, int t0, int ntok, const uint16_t* __restrict__ x,
+                                             const uint16_t* __restrict__ e_hi, const uint16_t* __restrict__ e_lo,
+                                             int32_t* __restrict__ labels, int n, int j, int jpad,
+                                             int2* __restrict__ changes, int32_t* __restrict__ nchanges,
+                                             const int32_t* __restrict__ lst) {
   const int bidx = blockIdx.y;
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
   const int h = lane / 32, l32 = lane % 32;
-  constexpr int kTokWave = 32 * NCB, kTokBlock = 4 * kTokWave;
-  const int tok0 = blockIdx.x * kTokBlock + wave * kTokWave;
-  const int ntok = LIST ? list_count[(size_t)bidx * kCounterStride] : n;  // positions < ntok hold tokens
-  if (LIST && (int)blockIdx.x * kTokBlock >= ntok) return;
-  const int32_t* lst = LIST ? list + (size_t)bidx * n : nullptr;
+  const int tok0 = t0 + wave * 32 * NCB;
   // token at position p of this block's range (positions past the range load a valid row, unused)
   auto token_at = [&](int pos) __attribute__((always_inline)) -> int {
     if constexpr (LIST)
@@ -651,6 +639,47 @@ cocluster_assign_kernel(const uint16_t* __restrict__ x, const uint16_t* __restri
       labels[(size_t)bidx * n + tokv[cb]] = lab[cb];
     }
     cpre += (int)__popcll(chm[cb]);
+  }
+}
+
+// Every token.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+cocluster_assign_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ e_hi,
+                        const uint16_t* __restrict__ e_lo, int32_t* __restrict__ labels, int n, int j, int jpad,
+                        int2* __restrict__ changes, int32_t* __restrict__ nchanges) {
+  __shared__ __attribute__((aligned(16))) AssignLds s_e;
+  assign_block<false, 4>(s_e, blockIdx.x * kAsgTok, n, x, e_hi, e_lo, labels, n, j, jpad, changes, nchanges, nullptr);
+}
+
+// The tokens that the certified fp16 pass or the candidate pass could not settle: per head b list[b][.], count[b]
+// entries.  Every block streams all of E, so what the lists hold in all decides the split.  Few tokens in blocks of four
+// column blocks per wave leave CUs idle beside a serial chain, and one column block per wave is faster (more blocks,
+// each a quarter of the MFMA work); many keep the E traffic down with four.
+// Measured (one column block against four, both sides' first pass, the key side's list of the stated length in all):
+// 12 heads x 32760 tokens, 500 clusters, 39 thousand listed 247 and 272 us, 157 thousand equal, 393 thousand 324 and
+// 309; 24 x 80000, 1000 clusters, 96 thousand 1024 and 1043 us, 192 thousand 1061 and 1052, all 1.9 million 1876 and
+// 1676.  (Of Gaussian tokens the certified pass leaves 7-15%, the candidate pass 0.6%; of tokens that are alike, with
+// clusters that are alike, all.)
+// MIXED: the lists may hold more than kFbShort tokens; each head goes by its own list times the heads.  Blocks past the
+// list exit at once.
+constexpr int kFbShort = 320 * kAsgTok;
+
+template <bool MIXED>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+cocluster_assign_list_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ e_hi,
+                             const uint16_t* __restrict__ e_lo, int32_t* __restrict__ labels, int n, int j, int jpad,
+                             int2* __restrict__ changes, int32_t* __restrict__ nchanges,
+                             const int32_t* __restrict__ list, const int32_t* __restrict__ list_count) {
+  __shared__ __attribute__((aligned(16))) AssignLds s_e;
+  const int ntok = list_count[(size_t)blockIdx.y * kCounterStride];
+  const int32_t* lst = list + (size_t)blockIdx.y * n;
+  if (!MIXED || (long long)ntok * gridDim.y <= kFbShort) {
+    if ((int)blockIdx.x * kAsgTokWave < ntok)
+      assign_block<true, 1>(s_e, blockIdx.x * kAsgTokWave, ntok, x, e_hi, e_lo, labels, n, j, jpad, changes, nchanges,
+                            lst);
+  } else if (MIXED && (int)blockIdx.x * kAsgTok < ntok) {
+    assign_block<true, MIXED ? 4 : 1>(s_e, blockIdx.x * kAsgTok, ntok, x, e_hi, e_lo, labels, n, j, jpad, changes,
+                                      nchanges, lst);
   }
 }
 
@@ -1742,24 +1771,25 @@ static int prep_launch(const uint16_t* a, const uint16_t* b, uint16_t* e_hi, uin
   return check_launch("svoo_cocluster_prep");
 }
 
-// short_list: the list is expected to be short (the candidate pass's leftovers, or the certified pass's of few
-// tokens): one column block per wave.
 static int assign_launch(const uint16_t* x, const uint16_t* e_hi, const uint16_t* e_lo, int32_t* labels, int bh, int n,
                          int j, int jpad, hipStream_t stream, int2* changes = nullptr, int32_t* nchanges = nullptr,
-                         const int32_t* list = nullptr, const int32_t* list_count = nullptr, bool short_list = false) {
-  if (list && short_list)
-    hipLaunchKernelGGL((cocluster_assign_kernel<true, 1>), dim3((n + 127) / 128, bh), dim3(256), 0, stream, x, e_hi,
-                       e_lo, labels, n, j, jpad, changes, nchanges, list, list_count);
-  else if (list)
-    hipLaunchKernelGGL((cocluster_assign_kernel<true, 4>), dim3((n + kAsgTok - 1) / kAsgTok, bh), dim3(256), 0, stream,
-                       x, e_hi, e_lo, labels, n, j, jpad, changes, nchanges, list, list_count);
-  else
-    hipLaunchKernelGGL((cocluster_assign_kernel<false, 4>), dim3((n + kAsgTok - 1) / kAsgTok, bh), dim3(256), 0,
-                       stream, x, e_hi, e_lo, labels, n, j, jpad, changes, nchanges, nullptr, nullptr);
+                         const int32_t* list = nullptr, const int32_t* list_count = nullptr) {
+  const dim3 grid((n + kAsgTok - 1) / kAsgTok, bh);
+  if (list) {
+    // one column block for lists of up to part tokens, as far as they can be that long, four for all n
+    const int part = kFbShort / bh;
+    const dim3 parts(max((int)grid.x, (min(n, part) + kAsgTokWave - 1) / kAsgTokWave), bh);
+    if (n <= part)
+      hipLaunchKernelGGL(cocluster_assign_list_kernel<false>, parts, dim3(256), 0, stream, x, e_hi, e_lo, labels, n, j,
+                         jpad, changes, nchanges, list, list_count);
+    else
+      hipLaunchKernelGGL(cocluster_assign_list_kernel<true>, parts, dim3(256), 0, stream, x, e_hi, e_lo, labels, n, j,
+                         jpad, changes, nchanges, list, list_count);
+  } else
+    hipLaunchKernelGGL(cocluster_assign_kernel, grid, dim3(256), 0, stream, x, e_hi, e_lo, labels, n, j, jpad, changes,
+                       nchanges);
   return check_launch("svoo_cocluster_assign");
 }
-
-static const long long kFbShortTokens = 1ll << 21;
 
 // The certified fp16 pass, then the hi + lo kernel on the tokens it left (fb_count must be zero on entry).
 // With bnd (and t_head) the pass records the pruning bounds; with list it runs on the listed tokens only.
@@ -1789,8 +1819,7 @@ static int assign16_launch(const uint16_t* x, const uint16_t* e16, const uint16_
                          nullptr);
   }
   if (int rc = check_launch("svoo_co_cluster (fp16 assign)")) return rc;
-  return assign_launch(x, e_hi, e_lo, labels, bh, n, j, jpad, stream, changes, nchanges, fb_list, fb_count,
-                       (long long)bh * n <= kFbShortTokens);
+  return assign_launch(x, e_hi, e_lo, labels, bh, n, j, jpad, stream, changes, nchanges, fb_list, fb_count);
 }
 
 static const int kMaxClusters = 4096;
@@ -2048,7 +2077,7 @@ extern "C" int svoo_co_cluster(const uint16_t* q, const uint16_t* k, int bh, int
         std::swap(t_prev, t_rec);
       }
       if ((r = check_launch("svoo_co_cluster (candidates)"))) return r;
-      r = assign_launch(x, e_hi, e_lo, labels, bh, n, kx, jpad, s, changes, cnt, fb_list, fb_count, true);
+      r = assign_launch(x, e_hi, e_lo, labels, bh, n, kx, jpad, s, changes, cnt, fb_list, fb_count);
     } else if (pr && !first) {
       hipLaunchKernelGGL(cocluster_prune_kernel, dim3((n + 256 * kPruneSub - 1) / (256 * kPruneSub), bh), dim3(256),
                          0, s, labels, bnd, delta, delta_max, n, jpad, plist, list_count);

@@ -238,6 +238,30 @@ def test_certified_fp16_pass_equals_hi_lo_labels(gpu, cfg_name, heads, zero01):
     assert torch.equal(r["klabels"], klab)
     assert torch.equal(r["qlabels"], qlab)
 
+
+@pytest.mark.parametrize("h,n", [(2, 5003), (2, 81920), (2, 81921), (2, 90001), (3, 60000)])
+def test_assignment_of_undecided_tokens(gpu, h, n):
+    """Lists of undecided tokens on both sides of the rule between one and four column blocks per wave (163840 tokens over
+    the heads): every cluster of head 0's keys comes twice, so that the first pass leaves all of its tokens (the lower
+    index wins), a third of the others' clusters do; the labels are those of the exact pass over every token."""
+    from svoo_amd.co_clustering import co_cluster_tokens_full, cocluster_assign
+
+    say("undecided tokens", h, n)
+    g = torch.Generator(device=gpu).manual_seed(n)
+    rn = lambda *s: torch.randn(*s, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
+    kc, qc, own = rn(h, 60, 128), rn(h, 20, 128), torch.arange(60, device=gpu)
+    src = torch.stack([torch.where(own < 60 - d, own, own - (60 - d)) for d in [30] + [20] * (h - 1)])
+    kc = torch.gather(kc, 1, src[..., None].expand(-1, -1, 128))
+    near = lambda c: (torch.gather(c, 1, torch.randint(0, c.shape[1], (h, n, 1), generator=g, device=gpu)  # noqa: E731
+                                   .expand(-1, -1, 128)) + 0.3 * rn(h, n, 128)).contiguous()
+    q, k = near(qc), near(kc)
+    r = co_cluster_tokens_full(q, k, 20, 60, 1, init_q_centroids=qc, init_k_centroids=kc)
+    klab = cocluster_assign(k, kc, qc)
+    assert torch.equal(r["klabels"], klab)
+    assert int(klab[0].max()) < 30 and int((r["ksizes"][0] > 0).sum()) <= 30
+    assert torch.equal(r["qlabels"], cocluster_assign(q, qc, r["kcentroids"]))
+
+
 def test_weighted_softmax_bit_exact(gpu):
     from svoo_amd.co_clustering import weighted_softmax
 
