@@ -504,9 +504,10 @@ __global__ void __launch_bounds__(kMaskThreads) block_mask_kernel(uint16_t* __re
 
 // The same row by one wave, E entries per lane (entry u * 64 + lane), without block barriers: a block of 256 threads per
 // row spent most of its time at some 17 of them and in wave 0's scans.  Differences from the block's kernel, none in a
-// result: the exponential comes from a table (within 1.3 units of the last place of float64, far below the rounding to
-// float32 and bf16) and the quotient from one reciprocal with a correction step, and a bin's count and mass share one
-// 32-bit LDS counter: a key of exponent e holds (128 + mantissa) 2^(e - 74) of the 2^60, so a bin's mass is a sum of
+// result: the exponential comes from a table (within 0.54 units of the last place of float64, the library's within 0.88)
+// and the quotient from one reciprocal with a correction step (the residual is exact and the reciprocal within 2^-53 of
+// itself, so it is within 0.5 + 2^-51 units; a division takes 1.8 us more at 4800 rows of 1000), and a bin's count and
+// mass share one 32-bit LDS counter: a key of exponent e holds (128 + mantissa) 2^(e - 74) of the 2^60, so a bin's mass is a sum of
 // integers below 2^18 times a power of two (below e = 74 each entry is rounded down on its own, as the mass demands).
 // The score and size loads are issued together on clamped indexes (a guarded load waits for the one before it: 11.7k of
 // a row's 46k cycles, then 1.7k).  What is left is the exact dots of the deferred scores (a third of a row: 25 of 1000
@@ -523,7 +524,7 @@ __global__ void __launch_bounds__(kMaskThreads) block_mask_wave_kernel(uint16_t*
                                                                        float p_st, uint8_t* __restrict__ map,
                                                                        int32_t* __restrict__ lengths) {
   constexpr int kW = kMaskThreads / kWave;
-  __shared__ double tab[64];
+  __shared__ double2 tab[64];
   __shared__ uint32_t hist_s[kW][2][kBins];
   __shared__ uint16_t dlist_s[kW][E * kWave], tfix_s[kW][E * kWave];
   const int tid = threadIdx.x, lane = tid % kWave;

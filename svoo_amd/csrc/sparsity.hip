@@ -40,7 +40,7 @@ __device__ __forceinline__ int sp_base(int w) { return (int)sp_raw((uint32_t)w *
 
 // float(exp(double(s - m))).  The library's exp costs about three times the instructions of exp_tab, and its constants,
 // kept in registers over the loop, spilled.  s <= m, or NaN.
-__device__ __forceinline__ float sp_weight(const double* exp2_tab, uint32_t raw, float scale, float m) {
+__device__ __forceinline__ float sp_weight(const double2* exp2_tab, uint32_t raw, float scale, float m) {
   const float s = __uint_as_float(raw << 16) * scale;
   return (float)exp_tab(exp2_tab, (double)(s - m));
 }
@@ -56,7 +56,7 @@ struct SpShared {
   uint32_t hist[32768];                // pattern b: 16 bits at half b & 1 of word b >> 1
   double mass[kSpGroups];              // per group of orders: the mass of its scores
   int32_t cnt[kSpGroups];              // and their number
-  double exp2_tab[64];                 // kExp2Table
+  double2 exp2_tab[64];                 // kExp2Table
   double wmass[kSpWaves];              // the same per wave's 64 groups
   int32_t wcnt[kSpWaves];
   uint16_t list[kSpGroups];            // non-empty groups, from the top

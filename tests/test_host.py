@@ -2,6 +2,7 @@
 
 import ctypes
 import re
+import subprocess
 from pathlib import Path
 
 import numpy as np
@@ -637,3 +638,43 @@ def test_exact_sparsity_rejects_bad_inputs():
         compute_exact_attention_sparsity(q.float(), q.float())
     with pytest.raises(ValueError):  # no CPU fallback: the counts run on the HIP device only
         compute_exact_attention_sparsity(q, q)
+
+
+def test_table_exponential_is_as_exact_as_the_library(tmp_path):
+    """The float64 exponential of the sparsity counts and the block mask, compiled for the host: within 0.54 units of the
+    last place of an 80-bit one (half a unit of the last addition, the polynomial's and the split's errors below a
+    sixteenth of |r| < 0.0055), where a device library's exp takes up to one."""
+    text = (ROOT / "svoo_amd" / "csrc" / "svoo_common.h").read_text()
+    part = text[text.index("// 2^(i / 64), i = 0"):text.index("// ---------------------------------------------------------------- wave scans")]
+    src = tmp_path / "exp.cpp"
+    src.write_text("""
+#include <cmath>
+#include <cstdint>
+struct double2 { double x, y; };
+#define __device__
+#define __forceinline__ inline
+""" + part + """
+extern "C" double worst(double scale, int n) {
+  double w = 0;
+  uint64_t s = 12345;
+  for (int i = 0; i < n; ++i) {
+    s = s * 6364136223846793005ull + 1442695040888963407ull;
+    const double x = -scale * (double)(s >> 11) * 0x1p-53;
+    const long double e = expl((long double)x);
+    int ex;
+    frexp((double)e, &ex);
+    w = fmax(w, (double)(fabsl((long double)exp_tab(kExp2Table, x) - e) / ldexpl(1.0L, ex - 53)));
+  }
+  return w;
+}
+extern "C" double one(double x) { return exp_tab(kExp2Table, x); }
+""")
+    lib = tmp_path / "exp.so"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-shared", "-fPIC", "-o", str(lib), str(src)], check=True)
+    h = ctypes.CDLL(str(lib))
+    h.worst.restype, h.worst.argtypes = ctypes.c_double, [ctypes.c_double, ctypes.c_int]
+    h.one.restype, h.one.argtypes = ctypes.c_double, [ctypes.c_double]
+    for scale in (200.0, 20.0, 1.0, 0.02):
+        assert h.worst(scale, 300000) < 0.54
+    assert h.one(0.0) == 1.0 and np.isnan(h.one(float("nan")))
+    assert 0.0 <= h.one(-1e30) < 1e-80 and h.one(float("-inf")) == h.one(-200.0)
