@@ -22,12 +22,16 @@ _MODULE_HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_ba
 
 def plain_execution() -> bool:
     """No tracing, compilation, function transform, forward-mode level, dispatch or function mode, or autocast: a kernel
-    launched on raw pointers then sees what the tensor operations would."""
-    return not (torch.jit.is_tracing() or torch.compiler.is_compiling()
-                or torch._C._functorch.peek_interpreter_stack() is not None
-                or torch.autograd.forward_ad._current_level >= 0
-                or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0
-                or torch.is_autocast_enabled("cuda"))
+    launched on raw pointers then sees what the tensor operations would.  Some of these can only be asked of names that
+    torch keeps to itself: where one is missing the answer is no."""
+    try:
+        return not (torch.jit.is_tracing() or torch.compiler.is_compiling()
+                    or torch._C._functorch.peek_interpreter_stack() is not None
+                    or torch.autograd.forward_ad._current_level >= 0
+                    or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0
+                    or torch.is_autocast_enabled("cuda"))
+    except (AttributeError, TypeError):
+        return False
 
 
 def _plain(t, dtype, device) -> bool:
@@ -38,7 +42,7 @@ def _plain(t, dtype, device) -> bool:
 def rms_norm_params(norm, width: int, device) -> Optional[tuple]:
     """``(weight or None, eps)`` when ``norm`` is exactly a ``torch.nn.RMSNorm`` over ``width`` elements whose call the
     kernel can stand in for (a bf16 weight, a given eps, no hooks or overridden forward), else None."""
-    if type(norm) is not torch.nn.RMSNorm or norm.normalized_shape != (width,) or norm.eps is None:
+    if type(norm) is not getattr(torch.nn, "RMSNorm", None) or norm.normalized_shape != (width,) or norm.eps is None:
         return None
     mod = torch.nn.modules.module
     if "forward" in norm.__dict__ or any(getattr(mod, n, None) for n in _GLOBAL_HOOKS) or \

@@ -678,3 +678,15 @@ extern "C" double one(double x) { return exp_tab(kExp2Table, x); }
         assert h.worst(scale, 300000) < 0.54
     assert h.one(0.0) == 1.0 and np.isnan(h.one(float("nan")))
     assert 0.0 <= h.one(-1e30) < 1e-80 and h.one(float("-inf")) == h.one(-200.0)
+
+
+@pytest.mark.parametrize("owner,name", [(torch._C._functorch, "peek_interpreter_stack"),
+                                        (torch.autograd.forward_ad, "_current_level"),
+                                        (torch._C, "_len_torch_dispatch_stack"), (torch._C, "_len_torch_function_stack")])
+def test_heads_pass_steps_aside_without_a_torch_name(monkeypatch, owner, name):
+    """A torch without one of the private names that the one-pass heads asks keeps the tensor operations."""
+    from svoo_amd import heads
+
+    assert heads.plain_execution()
+    monkeypatch.delattr(owner, name)
+    assert heads.plain_execution() is False
