@@ -55,8 +55,10 @@ def rms_norm_params(norm, width: int, device) -> Optional[tuple]:
 
 
 def rows_ok(x, heads: int) -> bool:
-    """``x [1, S, H*D]`` as rows the kernel reads: bf16, contiguous within a row, rows at 16-byte addresses."""
-    if type(x) not in (torch.Tensor, torch.nn.Parameter) or x.dim() != 3 or not x.is_cuda:
+    """``x [1, S, H*D]`` as rows the kernel reads: bf16, contiguous within a row, rows at 16-byte addresses, on the current
+    device (a launch goes to that one, also on another's null stream)."""
+    if type(x) not in (torch.Tensor, torch.nn.Parameter) or x.dim() != 3 or not x.is_cuda or \
+            x.device.index != torch.cuda.current_device():
         return False
     b, s, dim = x.shape
     return (b == 1 and s > 0 and heads > 0 and dim in (64 * heads, 128 * heads) and dim <= 8192

@@ -679,7 +679,7 @@ class Hunyuan_SAPAttn_Processor(WanAttn_SAPAttn_Processor):
             return heads.qkv_heads(query, key, value, h, **norm, **kw)
         # (the text's queries and keys are each normed where they have a norm; the pass takes both norms or none)
         text_norm = norm_args(("norm_added_q", "norm_added_k"))
-        if text_norm is None or text <= 0:
+        if text_norm is None or text <= 0 or encoder_hidden_states.device != query.device:
             return None
         projections = [getattr(attn, n, None) for n in ("add_q_proj", "add_k_proj", "add_v_proj")]
         if not all(heads.linear_ok(p, encoder_hidden_states, dim) for p in projections):

@@ -186,3 +186,17 @@ def test_the_operations_run_where_the_pass_cannot(gpu, monkeypatch):
         assert _heads(proc, layer, x, False, monkeypatch, **rope)[1] == 0
     type(proc).get_qk_norm = lambda self, attn, q, k: (q, k)
     assert _heads(proc, layer, x, False, monkeypatch, **rope)[1] == 0
+
+
+def test_rows_of_another_device_keep_the_operations(gpu, monkeypatch):
+    """Rows that are not on the current device: the tensor operations run, which go to their own."""
+    from svoo_amd import heads
+    from svoo_amd.processor import WanAttn_SAPAttn_Processor
+
+    say("heads: another device")
+    layer = Layer(2, 128, 256, gpu)
+    x = torch.randn(1, 40, 256, device=gpu, dtype=torch.bfloat16)
+    proc = _processor(WanAttn_SAPAttn_Processor)
+    assert heads.rows_ok(x, 2) and _heads(proc, layer, x, False, monkeypatch)[1] == 1
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: x.device.index + 1)
+    assert not heads.rows_ok(x, 2) and _heads(proc, layer, x, False, monkeypatch)[1] == 0
