@@ -803,8 +803,13 @@ class Hunyuan_SAPAttn_Processor(WanAttn_SAPAttn_Processor):
 
         # 1. Video part: cluster (or reuse), per-head ratios, block mask.
         self._mark("start")
-        # (views: a step that reuses the clustering reads neither, one that clusters makes them contiguous)
-        r = self.kmeans_clustering(query[:, :, :video_length], key[:, :, :video_length], self.layer_idx)
+        video = query[:, :, :video_length], key[:, :, :video_length]
+        # (a step that reuses the clustering reads neither: no copies)
+        if not self._uses_own(Hunyuan_SAPAttn_Processor, "kmeans_clustering", "should_recluster") or \
+                self.should_recluster():
+            video = tuple(t.contiguous() for t in video)
+        r = self.kmeans_clustering(*video, self.layer_idx)
+        del video
         self._mark("cluster")
         min_kc_ratio = self._get_min_kc_ratio_for_heads_from_step(self.current_inference_step, num_heads)
         q_sizes = r["qsizes"].view(cfg, num_heads, self.num_q_centroids)

@@ -690,3 +690,24 @@ def test_heads_pass_steps_aside_without_a_torch_name(monkeypatch, owner, name):
     assert heads.plain_execution()
     monkeypatch.delattr(owner, name)
     assert heads.plain_execution() is False
+
+
+@pytest.mark.parametrize("method", ["kmeans_clustering", "kmeans_init", "kmeans_step"])
+def test_hunyuan_clustering_methods_get_contiguous_video_tokens(method):
+    """A subclass that replaces a clustering method is given the video tokens as contiguous tensors."""
+    from svoo_amd.processor import Hunyuan_SAPAttn_Processor
+
+    class Stop(Exception):
+        pass
+
+    def replaced(self, query, key, layer_idx):
+        assert query.shape == key.shape == (1, 2, 12, 8)
+        assert query.is_contiguous() and key.is_contiguous()
+        raise Stop
+
+    cls = type("H", (Hunyuan_SAPAttn_Processor,), {
+        "prompt_length": 2, "context_length": 4, "num_frame": 3, "frame_size": 4, "first_times_fp": 1000,
+        "centroids_init": method == "kmeans_step", method: replaced})
+    q = torch.zeros(1, 2, 16, 8)
+    with pytest.raises(Stop):
+        cls(layer_idx=0).attention_core_logic(q, q.clone(), q.clone(), 500.0, 0)
