@@ -177,8 +177,18 @@ static inline __host__ __device__ int pm_kpp(int kp) { return (kp + kPmChunk - 1
 static inline __host__ __device__ size_t pm_praw_bytes(int kp) {
   return (size_t)kPmRows * (pm_kpp(kp) + 8) * sizeof(uint16_t);
 }
-static inline size_t pm_smem(int kp) {
-  return pm_praw_bytes(kp) + kPmRows * sizeof(double) + (size_t)2 * kPmChunk * kPmChunkStride * sizeof(uint16_t);
+static inline size_t pm_smem(int kp, int buffers) {
+  return pm_praw_bytes(kp) + kPmRows * sizeof(double) + (size_t)buffers * kPmChunk * kPmChunkStride * sizeof(uint16_t);
+}
+// B chunk buffers: two, unless the second costs a block per CU (of the three that the registers allow) that the launch
+// has blocks for.  One buffer -> two, standalone: 12 heads x 1000 clusters, 1000 columns 97.1 -> 102.6 us, 40 x 100,
+// 1408 columns 93 -> 119; where the same blocks fit or there are too few, two are 1-3% faster (12 x 100, 1000: 44.3 ->
+// 43.6).
+static int pm_buffers(int kp, long long blocks) {
+  constexpr size_t kLds = 160 * 1024;
+  constexpr long long kCus = 256;
+  const long long one = min((long long)(kLds / pm_smem(kp, 1)), 3ll), two = min((long long)(kLds / pm_smem(kp, 2)), 3ll);
+  return two < one && blocks > kCus * two ? 1 : 2;
 }
 
 // Element offset of E16[row][col] within a head: 32-row tiles of 8 KB, each [k-step 0..7][lane 0..63][8],
@@ -206,12 +216,13 @@ __global__ void __launch_bounds__(256) cocluster_prep_mfma_kernel(const uint16_t
                                                                   int32_t* __restrict__ t_out, int have_old,
                                                                   uint16_t* __restrict__ praw_out,
                                                                   double* __restrict__ inv_out,
-                                                                  float* __restrict__ nrm_out, double sqrt_kp) {
+                                                                  float* __restrict__ nrm_out, double sqrt_kp,
+                                                                  int buffers) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int kpp = pm_kpp(kp), ps = kpp + 8;
   uint16_t* praw = (uint16_t*)smem;                             // [16][ps] bf16
   double* inv = (double*)(smem + pm_praw_bytes(kp));           // [16]
-  uint16_t* bch = (uint16_t*)(inv + kPmRows);                   // [2][64][144] bf16
+  uint16_t* bch = (uint16_t*)(inv + kPmRows);                   // [buffers][64][144] bf16
   const int bidx = blockIdx.y, r0 = blockIdx.x * kPmRows;
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, li = lane % 16, q = lane / 16;
   const uint16_t* ab = a + (size_t)bidx * j * 128;
@@ -267,9 +278,15 @@ __global__ void __launch_bounds__(256) cocluster_prep_mfma_kernel(const uint16_t
   // Phase 2: inv = 1 / sqrt(sum + 1e-8), 16 threads per row.
   {
     const int r = tid / 16, sub = tid % 16;
-    // eight LDS reads in flight, summed in column order
+    // summed in column order; eight LDS reads in flight where there are more than four
     double sq = 0.0;
-    for (int k = sub; k < kp; k += 128) {
+    if (kp <= 64) {
+      for (int k = sub; k < kp; k += 16) {
+        const double v = (double)bf16_to_f32(praw[r * ps + k]);
+        sq += v * v;
+      }
+    }
+    for (int k = kp <= 64 ? kp : sub; k < kp; k += 128) {
       uint16_t p[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) p[i] = praw[r * ps + min(k + 16 * i, kpp - 1)];
@@ -320,9 +337,10 @@ __global__ void __launch_bounds__(256) cocluster_prep_mfma_kernel(const uint16_t
   const int poff = (lane % 16) * ps + 8 * (lane / 32);
   uint32_t bmax = 0;  // max |B| as bf16 magnitude bits (they order like the values)
   // Stage the chunk held in r (rows c ..) into buffer bch, request chunk c + 2 * kPmChunk into r, then the chunk's MFMAs.
-  // The two buffers alternate, so one barrier per chunk: a buffer is written again after the barrier of the chunk
-  // between, which every wave reaches with its reads of it done.
+  // Two buffers alternate, so one barrier per chunk: a buffer is written again after the barrier of the chunk between,
+  // which every wave reaches with its reads of it done.
   auto chunk_step = [&](u32x4_t(&r)[4], int c, uint16_t* bch) {
+    if (buffers == 1) __syncthreads();  // the previous chunk is consumed
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       *(u32x4_t*)(bch + (tid / 16 + 16 * i) * kPmChunkStride + (tid % 16) * 8) = r[i];
@@ -353,122 +371,130 @@ __global__ void __launch_bounds__(256) cocluster_prep_mfma_kernel(const uint16_t
   }
   for (int c = 0; c < kpp; c += 2 * kPmChunk) {
     chunk_step(pre0, c, bch);
-    if (c + kPmChunk < kpp) chunk_step(pre1, c + kPmChunk, bch + kPmChunk * kPmChunkStride);
+    if (c + kPmChunk < kpp) chunk_step(pre1, c + kPmChunk, bch + (buffers - 1) * kPmChunk * kPmChunkStride);
   }
   uint16_t* hb = e_hi + (size_t)bidx * jpad * 128;
   uint16_t* lb = e_lo + (size_t)bidx * jpad * 128;
+  // Lane l holds row r = l % 16 at columns dd0 + 8 (v / 4) + 4 (l / 32) + v % 4 (v = 0..15), lanes r and r + 16 the
+  // same values.  Slots 4q .. 4q + 3 are four consecutive columns: each array gets one 8-byte store per group (the fp64
+  // copy two 16-byte accesses) instead of four 2-byte (8-byte) ones.
+  const int rr = lane % 16, row = r0 + rr;
+  const bool upper = (lane & 16) != 0;
+  auto store_split = [&](int dd, const double(&ev)[4]) __attribute__((always_inline)) {
+    uint16_t hi[4], lo[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      hi[i] = f32_to_bf16((float)ev[i]);
+      lo[i] = f32_to_bf16((float)(ev[i] - (double)bf16_to_f32(hi[i])));
+    }
+    *(uint2*)(hb + (size_t)row * 128 + dd) = make_uint2(hi[0] | ((uint32_t)hi[1] << 16), hi[2] | ((uint32_t)hi[3] << 16));
+    *(uint2*)(lb + (size_t)row * 128 + dd) = make_uint2(lo[0] | ((uint32_t)lo[1] << 16), lo[2] | ((uint32_t)lo[3] << 16));
+  };
+  if (!e16) {
+    // hi and lo alone: by the lower lanes (shared by both, the 16 columns take 0.5 us longer in a launch of 7 to 14)
+    if (!upper && row < jpad) {
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        double ev[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ev[i] = (double)acc3[4 * q4 + i] * inv[rr];
+        store_split(dd0 + 8 * q4 + 4 * (lane / 32), ev);
+      }
+    }
+    return;
+  }
   // fp16 copy for the certified single-pass assignment: E * 2^t with one power of two per head, chosen
   // from an a-priori bound so that no element overflows (|E_ji| <= |P_j| |B_.i| <= sqrt(kp) max|B|, and
   // |P_j| <= 1): every block of the head derives the same t from max|B|.
   int t_scale = 0;
-  if (e16) {
-    __syncthreads();  // every thread is done with bch
-    uint32_t* red = (uint32_t*)bch;
-    for (int o = 32; o > 0; o >>= 1) bmax = max(bmax, (uint32_t)__shfl_xor((int)bmax, o));
-    if (lane == 0) red[wave] = bmax;
-    __syncthreads();
-    bmax = max(max(red[0], red[1]), max(red[2], red[3]));
-    __syncthreads();
-    if (bmax) {
-      int ex;
-      frexp(sqrt_kp * (double)bf16_to_f32((uint16_t)bmax), &ex);  // bound < 2^ex
-      t_scale = 15 - ex;
-    }
-    if (t_out && tid == 0) t_out[bidx] = t_scale;  // the same value from every block of the head
+  __syncthreads();  // every thread is done with bch
+  uint32_t* red = (uint32_t*)bch;
+  for (int o = 32; o > 0; o >>= 1) bmax = max(bmax, (uint32_t)__shfl_xor((int)bmax, o));
+  if (lane == 0) red[wave] = bmax;
+  __syncthreads();
+  bmax = max(max(red[0], red[1]), max(red[2], red[3]));
+  __syncthreads();
+  if (bmax) {
+    int ex;
+    frexp(sqrt_kp * (double)bf16_to_f32((uint16_t)bmax), &ex);  // bound < 2^ex
+    t_scale = 15 - ex;
   }
-  // Lane l holds row r = l % 16 at columns dd0 + 8 (v / 4) + 4 (l / 32) + v % 4 (v = 0..15), lanes r and r + 16 the
-  // same values: the first takes v < 8, the second the rest.
+  if (t_out && tid == 0) t_out[bidx] = t_scale;  // the same value from every block of the head
+  // The lower lanes take v < 8, the upper ones the rest.
   float err2 = 0.0f, nrm2 = 0.0f, dl2 = 0.0f;
-  const int rr = lane % 16, row = r0 + rr;
-  const bool upper = (lane & 16) != 0;
-  // Slots 4q .. 4q + 3 are four consecutive columns: each array gets one 8-byte store per group (the fp64 copy
-  // two 16-byte accesses) instead of four 2-byte (8-byte) ones.
   if (row < jpad) {
 #pragma unroll
     for (int qi = 0; qi < 2; ++qi) {
       const int dd = dd0 + 8 * (qi + (upper ? 2 : 0)) + 4 * (lane / 32);
-      uint16_t hi[4], lo[4], h16b[4];
+      uint16_t h16b[4];
       double ev[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float a3 = upper ? acc3[8 + 4 * qi + i] : acc3[4 * qi + i];
-        const double e = (double)a3 * inv[rr];
-        ev[i] = e;
-        hi[i] = f32_to_bf16((float)e);
-        lo[i] = f32_to_bf16((float)(e - (double)bf16_to_f32(hi[i])));
-      }
-      *(uint2*)(hb + (size_t)row * 128 + dd) =
-          make_uint2(hi[0] | ((uint32_t)hi[1] << 16), hi[2] | ((uint32_t)hi[3] << 16));
-      *(uint2*)(lb + (size_t)row * 128 + dd) =
-          make_uint2(lo[0] | ((uint32_t)lo[1] << 16), lo[2] | ((uint32_t)lo[3] << 16));
-      if (e16) {
-        double* eo = e_old ? e_old + ((size_t)bidx * jpad + row) * 128 + dd : nullptr;
+      for (int i = 0; i < 4; ++i) ev[i] = (double)(upper ? acc3[8 + 4 * qi + i] : acc3[4 * qi + i]) * inv[rr];
+      store_split(dd, ev);
+      double* eo = e_old ? e_old + ((size_t)bidx * jpad + row) * 128 + dd : nullptr;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          // padding rows (row >= j) are zero in the fp16 copy: their score is exactly 0
-          const double es = row < j ? ldexp(ev[i], t_scale) : 0.0;
-          const _Float16 h16 = (_Float16)(float)es;
-          const double err = es - (double)(float)h16;  // exact
-          err2 += (float)(err * err);
-          nrm2 += (float)((double)(float)h16 * (double)(float)h16);
-          h16b[i] = __builtin_bit_cast(uint16_t, h16);
-          if (eo && have_old) {
-            // change of E since the previous call on this buffer (for the pruning bounds)
-            const double df = ev[i] - old[qi][i];
-            dl2 += (float)(df * df);
-          }
+      for (int i = 0; i < 4; ++i) {
+        // padding rows (row >= j) are zero in the fp16 copy: their score is exactly 0
+        const double es = row < j ? ldexp(ev[i], t_scale) : 0.0;
+        const _Float16 h16 = (_Float16)(float)es;
+        const double err = es - (double)(float)h16;  // exact
+        err2 += (float)(err * err);
+        nrm2 += (float)((double)(float)h16 * (double)(float)h16);
+        h16b[i] = __builtin_bit_cast(uint16_t, h16);
+        if (eo && have_old) {
+          // change of E since the previous call on this buffer (for the pruning bounds)
+          const double df = ev[i] - old[qi][i];
+          dl2 += (float)(df * df);
         }
-        *(uint2*)(e16 + (size_t)bidx * jpad * 128 + e16_offset(row, dd)) =
-            make_uint2(h16b[0] | ((uint32_t)h16b[1] << 16), h16b[2] | ((uint32_t)h16b[3] << 16));
-        if (eo) {  // keep this E
-          *(double2*)eo = make_double2(ev[0], ev[1]);
-          *(double2*)(eo + 2) = make_double2(ev[2], ev[3]);
-        }
+      }
+      *(uint2*)(e16 + (size_t)bidx * jpad * 128 + e16_offset(row, dd)) =
+          make_uint2(h16b[0] | ((uint32_t)h16b[1] << 16), h16b[2] | ((uint32_t)h16b[3] << 16));
+      if (eo) {  // keep this E
+        *(double2*)eo = make_double2(ev[0], ev[1]);
+        *(double2*)(eo + 2) = make_double2(ev[2], ev[3]);
       }
     }
   }
-  if (e16) {
-    // Per-row |2^t E_j - E16_j| and |E16_j| (rows of real clusters only), then the head's maxima.  A row's 128
-    // columns are spread over lanes r, r + 16, r + 32 and r + 48 of each of the 4 waves.
-    err2 += __shfl_xor(err2, 16);
-    nrm2 += __shfl_xor(nrm2, 16);
-    dl2 += __shfl_xor(dl2, 16);
-    err2 += __shfl_xor(err2, 32);
-    nrm2 += __shfl_xor(nrm2, 32);
-    dl2 += __shfl_xor(dl2, 32);
-    float* part = (float*)bch;  // [wave][row][3]
-    __syncthreads();            // every wave is done with bch
-    if (lane < 16) {
-      part[(wave * 16 + lane) * 3] = err2;
-      part[(wave * 16 + lane) * 3 + 1] = nrm2;
-      part[(wave * 16 + lane) * 3 + 2] = dl2;
-    }
-    __syncthreads();
-    if (tid < 16) {
-      const int i = tid;
-      float er = 0.0f, nr = 0.0f, dl = 0.0f;
-      if (r0 + i < j)
-        for (int w = 0; w < 4; ++w) {
-          er += part[(w * 16 + i) * 3];
-          nr += part[(w * 16 + i) * 3 + 1];
-          dl += part[(w * 16 + i) * 3 + 2];
-        }
-      // rounded-to-nearest fp32 sums of at most 128 squares: 2^-17 relative slack covers their rounding
-      er = sqrtf(er * (1.0f + 0x1p-16f)) * (1.0f + 0x1p-20f);
-      nr = sqrtf(nr * (1.0f + 0x1p-16f)) * (1.0f + 0x1p-20f);
-      dl = sqrtf(dl * (1.0f + 0x1p-16f)) * (1.0f + 0x1p-20f);
-      if (e_old && have_old && r0 + i < jpad) delta[(size_t)bidx * jpad + r0 + i] = dl;
+  // Per-row |2^t E_j - E16_j| and |E16_j| (rows of real clusters only), then the head's maxima.  A row's 128
+  // columns are spread over lanes r, r + 16, r + 32 and r + 48 of each of the 4 waves.
+  err2 += __shfl_xor(err2, 16);
+  nrm2 += __shfl_xor(nrm2, 16);
+  dl2 += __shfl_xor(dl2, 16);
+  err2 += __shfl_xor(err2, 32);
+  nrm2 += __shfl_xor(nrm2, 32);
+  dl2 += __shfl_xor(dl2, 32);
+  float* part = (float*)bch;  // [wave][row][3]
+  __syncthreads();            // every wave is done with bch
+  if (lane < 16) {
+    part[(wave * 16 + lane) * 3] = err2;
+    part[(wave * 16 + lane) * 3 + 1] = nrm2;
+    part[(wave * 16 + lane) * 3 + 2] = dl2;
+  }
+  __syncthreads();
+  if (tid < 16) {
+    const int i = tid;
+    float er = 0.0f, nr = 0.0f, dl = 0.0f;
+    if (r0 + i < j)
+      for (int w = 0; w < 4; ++w) {
+        er += part[(w * 16 + i) * 3];
+        nr += part[(w * 16 + i) * 3 + 1];
+        dl += part[(w * 16 + i) * 3 + 2];
+      }
+    // rounded-to-nearest fp32 sums of at most 128 squares: 2^-17 relative slack covers their rounding
+    er = sqrtf(er * (1.0f + 0x1p-16f)) * (1.0f + 0x1p-20f);
+    nr = sqrtf(nr * (1.0f + 0x1p-16f)) * (1.0f + 0x1p-20f);
+    dl = sqrtf(dl * (1.0f + 0x1p-16f)) * (1.0f + 0x1p-20f);
+    if (e_old && have_old && r0 + i < jpad) delta[(size_t)bidx * jpad + r0 + i] = dl;
 #pragma unroll
-      for (int o = 8; o > 0; o >>= 1) {
-        er = fmaxf(er, __shfl_xor(er, o));
-        nr = fmaxf(nr, __shfl_xor(nr, o));
-        dl = fmaxf(dl, __shfl_xor(dl, o));
-      }
-      if (tid == 0) {
-        atomicMax(err_max + bidx, __float_as_uint(er));
-        atomicMax(norm_max + bidx, __float_as_uint(nr));
-        if (e_old && have_old) atomicMax(delta_max + bidx, __float_as_uint(dl));
-      }
+    for (int o = 8; o > 0; o >>= 1) {
+      er = fmaxf(er, __shfl_xor(er, o));
+      nr = fmaxf(nr, __shfl_xor(nr, o));
+      dl = fmaxf(dl, __shfl_xor(dl, o));
+    }
+    if (tid == 0) {
+      atomicMax(err_max + bidx, __float_as_uint(er));
+      atomicMax(norm_max + bidx, __float_as_uint(nr));
+      if (e_old && have_old) atomicMax(delta_max + bidx, __float_as_uint(dl));
     }
   }
 }
@@ -1755,9 +1781,10 @@ static int prep_launch(const uint16_t* a, const uint16_t* b, uint16_t* e_hi, uin
                        int have_old = 0, uint16_t* praw_out = nullptr, double* inv_out = nullptr,
                        float* nrm_out = nullptr) {
   if (kp <= kPmMaxKp) {
-    hipLaunchKernelGGL(cocluster_prep_mfma_kernel, dim3(jpad / kPmRows, bh), dim3(256), pm_smem(kp), stream, a, b,
-                       e_hi, e_lo, profile, j, kp, jpad, e16, err_max, norm_max, e_old, delta, delta_max, t_out,
-                       have_old, praw_out, inv_out, nrm_out, sqrt((double)kp));
+    const int buffers = pm_buffers(kp, (long long)(jpad / kPmRows) * bh);
+    hipLaunchKernelGGL(cocluster_prep_mfma_kernel, dim3(jpad / kPmRows, bh), dim3(256), pm_smem(kp, buffers), stream, a,
+                       b, e_hi, e_lo, profile, j, kp, jpad, e16, err_max, norm_max, e_old, delta, delta_max, t_out,
+                       have_old, praw_out, inv_out, nrm_out, sqrt((double)kp), buffers);
     return check_launch("svoo_cocluster_prep");
   }
   // Wide profiles: the vector kernel.  Few rows -> 2 rows per block for more blocks; many -> 8.

@@ -239,6 +239,29 @@ def test_certified_fp16_pass_equals_hi_lo_labels(gpu, cfg_name, heads, zero01):
     assert torch.equal(r["qlabels"], qlab)
 
 
+@pytest.mark.parametrize("heads,j,kp", [(40, 100, 16), (40, 100, 64), (40, 100, 65), (40, 290, 600), (11, 1000, 1000),
+                                        (40, 100, 1408)])
+def test_profiles_of_many_heads_at_once(gpu, heads, j, kp):
+    """Profile widths around the norm's loops, and launches of more blocks than fit at once, where the products' chunks go
+    through one buffer where a second would cost a block per CU: every head's P and E are those of the head alone (two
+    buffers)."""
+    from svoo_amd.co_clustering import cocluster_profile
+
+    say("profiles of many heads", heads, j, kp)
+    _, a = rand_bf16((heads, j, 128), kp, gpu)
+    _, b = rand_bf16((heads, kp, 128), kp + 1, gpu)
+    got = cocluster_profile(a, b)
+    for i in (0, heads // 2, heads - 1):
+        for g, w in zip(got, cocluster_profile(a[i : i + 1].contiguous(), b[i : i + 1].contiguous())):
+            assert torch.equal(g[i], w[0])
+    # P against its definition: bf16(A B^T) exact to its rounding (1 bf16 step at a midpoint of the fp64 sums), fp32
+    i = heads - 1
+    dots = (a[i].double() @ b[i].double().T).float().to(torch.bfloat16).double()
+    want = dots / (dots.square().sum(-1, keepdim=True) + 1e-8).sqrt()
+    assert ((got[0][i].double() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -23).all()
+    assert (got[0][i].double() - want).norm() <= 1e-4 * want.norm()
+
+
 @pytest.mark.parametrize("h,n", [(2, 5003), (2, 81920), (2, 81921), (2, 90001), (3, 60000)])
 def test_assignment_of_undecided_tokens(gpu, h, n):
     """Lists of undecided tokens on both sides of the rule between one and four column blocks per wave (163840 tokens over
