@@ -188,6 +188,43 @@ def test_the_operations_run_where_the_pass_cannot(gpu, monkeypatch):
     assert _heads(proc, layer, x, False, monkeypatch, **rope)[1] == 0
 
 
+@pytest.mark.parametrize("norm_width", [256, 128])
+def test_heads_of_non_finite_rows(gpu, monkeypatch, norm_width):
+    """Rows with +inf, -inf, NaN and the type's largest values: NaN where the operations give NaN, the same values
+    elsewhere (norm over the row, whose sum overflows, and per head)."""
+    from svoo_amd.processor import Hunyuan_SAPAttn_Processor, WanAttn_SAPAttn_Processor
+
+    say("heads: non-finite rows", norm_width)
+    torch.manual_seed(2)
+    wan = norm_width == 256
+    layer = Layer(2, 128, norm_width, gpu)
+    for n in ("to_q", "to_k", "to_v"):
+        setattr(layer, n, torch.nn.Identity())  # the rows themselves
+    x = torch.randn(1, 9, 256, device=gpu, dtype=torch.bfloat16)
+    x[0, 1, 3], x[0, 2, 200], x[0, 3, 7], x[0, 4, 130], x[0, 5] = np.inf, -np.inf, np.nan, 3.0e38, 0.0
+    x[0, 6, :128] = np.nan
+    cos, sin = _tables(9, 128, gpu)
+    kw = dict(rotary_emb=(cos[None, :, None], sin[None, :, None])) if wan else dict(image_rotary_emb=(cos, sin))
+    proc = _processor(WanAttn_SAPAttn_Processor if wan else Hunyuan_SAPAttn_Processor)
+    for norms in (True, False):
+        if not norms:
+            layer.norm_q = layer.norm_k = None
+        want, _ = _heads(proc, layer, x, True, monkeypatch, **kw)
+        got, n = _heads(proc, layer, x, False, monkeypatch, **kw)
+        assert n == 1
+        for g, w in zip(got, want):
+            assert torch.equal(g.isnan(), w.isnan()) and torch.equal(g.isinf(), w.isinf())
+        clean = lambda ts: [t.nan_to_num(0.0, 1.0, -1.0) for t in ts]  # noqa: E731
+        g, w = clean(got), clean(want)
+        assert torch.equal(g[2], w[2])
+        if norms:
+            for a, b in zip(g[:2], w[:2]):  # one bf16 step of either of the pair, as in _close
+                pair = b.double().unflatten(-1, (-1, 2)).abs().sum(-1, keepdim=True).expand(-1, -1, -1, -1, 2).flatten(-2)
+                assert ((a.double() - b.double()).abs() <= 2.0 ** -6 * pair + 1e-30).all()
+        else:
+            assert torch.equal(g[0], w[0]) and torch.equal(g[1], w[1])
+
+
 def test_rows_of_another_device_keep_the_operations(gpu, monkeypatch):
     """Rows that are not on the current device: the tensor operations run, which go to their own."""
     from svoo_amd import heads

@@ -54,6 +54,26 @@ def test_library_reports_errors_without_launching():
     assert L.svoo_convert(1, 2, 1, 0, 0, None) == 0  # nothing to convert: no launch
 
 
+@pytest.mark.parametrize("change,code,message", [
+    (dict(d=96), -2, "D=96"), (dict(d=32), -2, "D=32"), (dict(heads=65), -2, "above 8192"), (dict(heads=0), -2, "H=0"),
+    (dict(q=None), -1, "null pointer"), (dict(v_out=None), -1, "null pointer"), (dict(rows=0), -1, "rows=0"),
+    (dict(out_row0=1), -1, "rows=4 at 1 of 4"), (dict(out_row0=-1), -1, "rows=4 at -1"), (dict(norm=3), -1, "norm=3"),
+    (dict(form=2), -1, "rope_form=2"), (dict(cos=16), -1, "rope tables"), (dict(cos=16, sin=16, rope_rows=5), -1, "5 rows"),
+    (dict(k=8), -1, "16-byte"), (dict(v_stride=12), -1, "16-byte"), (dict(q_weight=2), -1, "16-byte"),
+])
+def test_heads_entry_refuses_what_its_kernel_does_not_take(change, code, message):
+    """Widths, head dims, row ranges and addresses outside svoo_qkv_heads' contract: refused before any launch."""
+    from svoo_amd import _lib
+
+    a = dict(q=16, k=16, v=16, q_stride=8192, k_stride=8192, v_stride=8192, q_out=16, k_out=16, v_out=16, rows=4, heads=2,
+             d=128, out_rows=4, out_row0=0, norm=0, q_weight=None, k_weight=None, q_eps=0.0, k_eps=0.0, cos=None, sin=None,
+             rope_rows=0, form=0)
+    assert set(change) <= set(a)
+    a.update(change)
+    assert _lib.lib().svoo_qkv_heads(*a.values(), None) == code
+    assert message in _lib.last_error(), _lib.last_error()
+
+
 def test_operators_reject_non_float_inputs_before_any_call():
     """Operands are bf16, fp16 or fp32 (fp16 / fp32 are rounded to bf16 on the GPU); anything else is refused
     on the host, before a GPU is touched."""
