@@ -244,8 +244,9 @@ int svoo_vbsa_fused_fwd_noalloc(const uint16_t* q, const uint16_t* k, const uint
  *     svoo/co_clustering.py:1692-1797.
  *   svoo_vbsa_ear_fwd: for each (b, i), softmax attention of Q_i over the tokens of the active key
  *     clusters and the (k_cent_j, v_cent_j) pairs of the inactive ones, scored
- *     q . k_cent_j / sqrt(D) + log(|K_j| + 1e-6): one online softmax (fp32, bf16 MFMA).  Workspace and
- *     status as svoo_vbsa_fwd.  Replaces dynamic_block_sparse_prune_fwd_flashinfer (FlashInfer
+ *     q . k_cent_j / sqrt(D) + log(|K_j| + 1e-6): one online softmax (fp32, bf16 MFMA).  k_cent and v_cent lie a
+ *     multiple of 256 bytes, and fewer than 2^31 - B*H*(N + KN) rows of 256 bytes, from k and v; other buffers are
+ *     refused.  Workspace and status as svoo_vbsa_fwd.  Replaces dynamic_block_sparse_prune_fwd_flashinfer (FlashInfer
  *     attention with return_lse + _fused_qc_kernel_opt), svoo/co_clustering.py:1801-2050.
  * ------------------------------------------------------------------------------------------- */
 int svoo_ear_value_stats(const uint16_t* v_perm, const int32_t* k_offsets, const int32_t* k_sizes, int bh, int n,

@@ -2147,7 +2147,7 @@ extern "C" int svoo_co_cluster(const uint16_t* q, const uint16_t* k, int bh, int
       break;
   }
   // The stable sort of the final labels (the first iteration's sort already is when max_iters == 1).
-  // The two sides' final sorts are independent: one set of three launches, the query side's counts in the change
+  // The two sides' final sorts are independent: one set of launches, the query side's counts in the change
   // list's buffer (consumed by now); their sorted labels are not needed.
   if (rc == SVOO_OK && max_iters > 1) {
     if (svoo_cluster_sort_workspace_size(bh, n, qc) <= (size_t)bh * n * sizeof(int2)) {

@@ -28,7 +28,7 @@ constexpr int kSortChunk = 1024;
 constexpr int kMaxSortClusters = 16384;
 
 // One sort of a launch: a launch sorts the rows of one or two of them (rows [0, bh_a) the first, the rest the
-// second), so that two independent sorts share their three launches.
+// second), so that two independent sorts share their launches.
 struct SortSide {
   const int32_t* labels;
   int32_t* counts;
@@ -189,6 +189,8 @@ constexpr int kSortSmallN = 12288;
 constexpr int kSortSmallK = 1024;
 constexpr int kSortSmallThreads = 1024;
 constexpr int kSortSmallWaves = kSortSmallThreads / kWave;
+static_assert(kSortSmallN % kSortSmallThreads == 0, "a wave's tokens fill its kRounds registers at most");
+static_assert(kSortSmallK <= kSortSmallThreads, "one thread per cluster scans the waves' counts");
 
 // One block per row: the three passes in one launch (k <= kSortSmallK, n <= kSortSmallN; LDS int32 [16][k]).
 __global__ void __launch_bounds__(kSortSmallThreads) sort_small_kernel(SortSide sa, SortSide sb, int bh_a, int n,
@@ -207,7 +209,7 @@ __global__ void __launch_bounds__(kSortSmallThreads) sort_small_kernel(SortSide 
   const int b = second ? blockIdx.x - bh_a : blockIdx.x, k = S.k;
   for (int i = tid; i < kSortSmallWaves * k; i += kSortSmallThreads) hist[i] = 0;
   __syncthreads();
-  // the wave's tokens: `rounds` groups of 64, at most 16, all in registers
+  // the wave's tokens: `rounds` groups of 64, at most kRounds (12), all in registers
   const int rounds = ((n + kWave - 1) / kWave + kSortSmallWaves - 1) / kSortSmallWaves;
   const int t0 = wave * rounds * kWave;
   const int32_t* lab = S.labels + (size_t)b * n;
@@ -291,10 +293,6 @@ extern "C" size_t svoo_cluster_sort_workspace_size(int bh, int n, int k) {
   return ((size_t)bh * k * sort_nchunks(n) * sizeof(int32_t) + 255) / 256 * 256 + 256;
 }
 
-// Internal entry used by the co-clustering driver: the workspace pointer is already sized.
-// With a guard the three kernels do their work only when *guard > limit (a count on the device; the
-// co-clustering's choice between a full recount and the incremental update); then the histogram pass also
-// clears zn doubles at zero_sums when given.
 static SortSide sort_side(const int32_t* labels, int k, int32_t* sorted_idx, int32_t* sizes, int32_t* offsets,
                           int32_t* sorted_labels, int32_t* counts) {
   int kbits = 0;
@@ -322,9 +320,9 @@ static int sort_launch(const SortSide& sa, const SortSide& sb, int bh_a, int bh_
 }
 
 // Internal entry used by the co-clustering driver: the workspace pointer is already sized.
-// With a guard the three kernels do their work only when *guard > limit (a count on the device; the
-// co-clustering's choice between a full recount and the incremental update); then the histogram pass also
-// clears zn doubles at zero_sums when given.
+// With a guard the kernels do their work only when *guard > limit (a count on the device; the co-clustering's choice
+// between a full recount and the incremental update); then the first of them also clears zn doubles at zero_sums when
+// given.
 int svoo_cluster_sort_impl(const int32_t* labels, int bh, int n, int k, int32_t* sorted_idx, int32_t* sizes,
                            int32_t* offsets, int32_t* sorted_labels, int32_t* counts, int32_t* err,
                            hipStream_t stream, const int32_t* guard, int limit, double* zero_sums, long long zero_n) {
@@ -332,7 +330,7 @@ int svoo_cluster_sort_impl(const int32_t* labels, int bh, int n, int k, int32_t*
   return sort_launch(sa, sa, bh, 0, n, err, stream, guard, limit, zero_sums, zero_n);
 }
 
-// Two independent sorts of bh rows each (their own counts workspaces) in one set of three launches.
+// Two independent sorts of bh rows each (their own counts workspaces) in one set of launches (three, or one of short rows).
 int svoo_cluster_sort2_impl(const int32_t* labels_a, int k_a, int32_t* sorted_idx_a, int32_t* sizes_a,
                             int32_t* offsets_a, int32_t* sorted_labels_a, int32_t* counts_a, const int32_t* labels_b,
                             int k_b, int32_t* sorted_idx_b, int32_t* sizes_b, int32_t* offsets_b,

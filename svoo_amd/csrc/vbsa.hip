@@ -1336,14 +1336,15 @@ int vbsa_launch(const char* name, const uint16_t* q, const uint16_t* k, const ui
   SVOO_REQUIRE(workspace && ws_bytes >= lay.total, SVOO_ERR_WORKSPACE, "%s: workspace %zu < %zu", name, ws_bytes,
                lay.total);
   if (EAR) {
-    // the entry's contract on where the centroid buffers lie
+    // What the entry refuses (stated in the header).  The kernel needs less: each tile's copies go from a base of their
+    // own, and 16-byte addresses are enough.
     const long long dk = (long long)(uintptr_t)kc - (long long)(uintptr_t)k;
     const long long dv = (long long)(uintptr_t)vc - (long long)(uintptr_t)v;
     SVOO_REQUIRE(dk % 256 == 0 && dv % 256 == 0, SVOO_ERR_INVALID_ARG,
                  "%s: centroid buffers must be 256-byte congruent with k and v", name);
     const long long lim = (1ll << 31) - 1 - (long long)bh * (s + kn);
     SVOO_REQUIRE(llabs(dk / 256) < lim && llabs(dv / 256) < lim, SVOO_ERR_UNSUPPORTED,
-                 "%s: centroid buffers too far from k / v for int32 row offsets", name);
+                 "%s: centroid buffers too far from k / v (2^31 rows of 256 bytes)", name);
   }
   hipStream_t st = (hipStream_t)stream;
   char* base = (char*)workspace;

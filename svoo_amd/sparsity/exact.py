@@ -29,8 +29,8 @@ DEFAULT_SPARSITY_THRESHOLD = 0.95
 # Share of the device's free memory one query chunk's bf16 scores may take when the chunk is sized
 # automatically; SVOO_SPARSITY_AUTO_MEM_FRACTION overrides it (the reference's knob, same meaning).
 DEFAULT_AUTO_MEMORY_FRACTION = 0.45
-# Above this many score bytes per chunk the count kernel, not the GEMM launch count, sets the time,
-# so larger chunks buy nothing and only hold memory.
+# Above this many score bytes per chunk the products and the counts themselves, not the number of their launches, set
+# the time, so larger chunks buy nothing and only hold memory.
 _MAX_CHUNK_SCORE_BYTES = 4 << 30
 _SCORE_BYTES = 2  # bf16 scores; the counts need no per-score scratch
 _SPARSITY_HEADER_RE = re.compile(r"\[Sparsity\] Layer (\d+) \| Type: \w+ \| Step: (\d+)")
