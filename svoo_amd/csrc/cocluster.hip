@@ -684,11 +684,14 @@ cocluster_assign_kernel(const uint16_t* __restrict__ x, const uint16_t* __restri
 // Measured (one column block against four, both sides' first pass, the key side's list of the stated length in all):
 // 12 heads x 32760 tokens, 500 clusters, 39 thousand listed 247 and 272 us, 157 thousand equal, 393 thousand 324 and
 // 309; 24 x 80000, 1000 clusters, 96 thousand 1024 and 1043 us, 192 thousand 1061 and 1052, all 1.9 million 1876 and
-// 1676.  (Of Gaussian tokens the certified pass leaves 7-15%, the candidate pass 0.6%; of tokens that are alike, with
-// clusters that are alike, all.)
-// MIXED: the lists may hold more than kFbShort tokens; each head goes by its own list times the heads.  Blocks past the
-// list exit at once.
-constexpr int kFbShort = 320 * kAsgTok;
+// 1676; the key passes of a Wan 1.3B step, 110-204 thousand over 12 heads that differ, 86 and 96 a launch.  (Of Gaussian
+// tokens the certified pass leaves 7-15%, the candidate pass 0.6%; of tokens that are alike, with clusters that are
+// alike, all.)
+// MIXED: the lists may hold more than kFbShort tokens.  A head whose list would not fill its share of them knows it is
+// short; one with more asks for the sum over the heads (by its own list alone the first key pass of a Wan 1.3B step,
+// whose heads differ, took 103 us instead of 90; asked by every block, 0.5 us a launch).  Blocks past the list exit at
+// once.
+constexpr int kFbShort = 416 * kAsgTok;
 
 template <bool MIXED>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -699,10 +702,20 @@ cocluster_assign_list_kernel(const uint16_t* __restrict__ x, const uint16_t* __r
   __shared__ __attribute__((aligned(16))) AssignLds s_e;
   const int ntok = list_count[(size_t)blockIdx.y * kCounterStride];
   const int32_t* lst = list + (size_t)blockIdx.y * n;
-  if (!MIXED || (long long)ntok * gridDim.y <= kFbShort) {
-    if ((int)blockIdx.x * kAsgTokWave < ntok)
-      assign_block<true, 1>(s_e, blockIdx.x * kAsgTokWave, ntok, x, e_hi, e_lo, labels, n, j, jpad, changes, nchanges,
-                            lst);
+  const int first = blockIdx.x * kAsgTokWave;
+  if (first >= ntok) return;
+  bool short_lists = true;
+  if (MIXED && (long long)ntok * gridDim.y > kFbShort) {  // longer than the heads' mean could be
+    int total = 0;
+    for (unsigned b = threadIdx.x % kWave; b < gridDim.y; b += kWave) total += list_count[(size_t)b * kCounterStride];
+    short_lists = __builtin_amdgcn_readlane(wave_scan_i32(total), kWave - 1) <= kFbShort;
+  }
+  if (short_lists) {
+    for (int t0 = first; t0 < ntok; t0 += gridDim.x * kAsgTokWave) {
+      if (t0 != first) __syncthreads();  // the last part's chunks are consumed
+      assign_block<true, 1>(s_e, t0, ntok, x, e_hi, e_lo, labels, n, j, jpad, changes, nchanges, lst);
+      if (!MIXED) break;  // (its grid has a block for every part)
+    }
   } else if (MIXED && (int)blockIdx.x * kAsgTok < ntok) {
     assign_block<true, MIXED ? 4 : 1>(s_e, blockIdx.x * kAsgTok, ntok, x, e_hi, e_lo, labels, n, j, jpad, changes,
                                       nchanges, lst);
@@ -1803,9 +1816,9 @@ static int assign_launch(const uint16_t* x, const uint16_t* e_hi, const uint16_t
                          const int32_t* list = nullptr, const int32_t* list_count = nullptr) {
   const dim3 grid((n + kAsgTok - 1) / kAsgTok, bh);
   if (list) {
-    // one column block for lists of up to part tokens, as far as they can be that long, four for all n
+    // blocks for lists of twice the heads' mean by one column block (longer ones loop) and of n by four
     const int part = kFbShort / bh;
-    const dim3 parts(max((int)grid.x, (min(n, part) + kAsgTokWave - 1) / kAsgTokWave), bh);
+    const dim3 parts(max((int)grid.x, (min(n, 2 * part) + kAsgTokWave - 1) / kAsgTokWave), bh);
     if (n <= part)
       hipLaunchKernelGGL(cocluster_assign_list_kernel<false>, parts, dim3(256), 0, stream, x, e_hi, e_lo, labels, n, j,
                          jpad, changes, nchanges, list, list_count);

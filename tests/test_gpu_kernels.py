@@ -262,18 +262,20 @@ def test_profiles_of_many_heads_at_once(gpu, heads, j, kp):
     assert (got[0][i].double() - want).norm() <= 1e-4 * want.norm()
 
 
-@pytest.mark.parametrize("h,n", [(2, 5003), (2, 81920), (2, 81921), (2, 90001), (3, 60000)])
-def test_assignment_of_undecided_tokens(gpu, h, n):
-    """Lists of undecided tokens on both sides of the rule between one and four column blocks per wave (163840 tokens over
+@pytest.mark.parametrize("h,n,others", [(2, 5003, 20), (2, 106496, 20), (2, 106497, 20), (2, 120001, 30), (3, 80000, 20),
+                                        (8, 60000, 0)])
+def test_assignment_of_undecided_tokens(gpu, h, n, others):
+    """Lists of undecided tokens on both sides of the rule between one and four column blocks per wave (212992 tokens over
     the heads): every cluster of head 0's keys comes twice, so that the first pass leaves all of its tokens (the lower
-    index wins), a third of the others' clusters do; the labels are those of the exact pass over every token."""
+    index wins), and ``others`` of 60 - others clusters in the other heads (none: head 0's list is short in all, longer
+    than its grid's blocks); the labels are those of the exact pass over every token."""
     from svoo_amd.co_clustering import co_cluster_tokens_full, cocluster_assign
 
-    say("undecided tokens", h, n)
+    say("undecided tokens", h, n, others)
     g = torch.Generator(device=gpu).manual_seed(n)
     rn = lambda *s: torch.randn(*s, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
     kc, qc, own = rn(h, 60, 128), rn(h, 20, 128), torch.arange(60, device=gpu)
-    src = torch.stack([torch.where(own < 60 - d, own, own - (60 - d)) for d in [30] + [20] * (h - 1)])
+    src = torch.stack([torch.where(own < 60 - d, own, own - (60 - d)) for d in [30] + [others] * (h - 1)])
     kc = torch.gather(kc, 1, src[..., None].expand(-1, -1, 128))
     near = lambda c: (torch.gather(c, 1, torch.randint(0, c.shape[1], (h, n, 1), generator=g, device=gpu)  # noqa: E731
                                    .expand(-1, -1, 128)) + 0.3 * rn(h, n, 128)).contiguous()
