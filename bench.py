@@ -419,7 +419,7 @@ def kernel_table(step, cfg, h, nv, d, qcn, kcn, iters):
     # Passes of the co-clustering, in launch order: each starts with its prep kernel and alternates key side,
     # query side.  A key-side pass from the second iteration on is the candidate pass (radius, lists, score
     # kernels) when the library takes it, else the full pass; each ends with the hi/lo kernel on the tokens it
-    # left (cocluster_assign_kernel).
+    # left (cocluster_assign_list_kernel).
     passes = []
     for e in evs:
         nm = short(e.name)
@@ -430,9 +430,9 @@ def kernel_table(step, cfg, h, nv, d, qcn, kcn, iters):
     tot = lambda pz, names: sum(sum(pz["k"].get(nm, [])) for nm in names)  # noqa: E731
     key_passes = [pz for pz in passes if pz["side"] == "key"]
     qry_passes = [pz for pz in passes if pz["side"] == "query"]
-    full_names = ("cocluster_assign16_kernel", "cocluster_assign_kernel")
+    full_names = ("cocluster_assign16_kernel", "cocluster_assign_list_kernel")
     cand_names = ("cocluster_nu_kernel", "cocluster_radius_kernel", "cocluster_lists_kernel",
-                  "cocluster_score_kernel", "cocluster_assign_kernel")
+                  "cocluster_score_kernel", "cocluster_assign_list_kernel")
     if key_passes and "cocluster_assign16_kernel" in key_passes[0]["k"]:
         # the first key-side pass scores every cluster for every token: its MFMA roofline
         key_us = tot(key_passes[0], full_names)
@@ -441,7 +441,7 @@ def kernel_table(step, cfg, h, nv, d, qcn, kcn, iters):
                                     "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                                     "frac": round(key_flop / (key_us * 1e-6) / 1e12 / BF16_PEAK_TFLOPS, 4),
                                     "full_pass_us": round(key_us, 2),
-                                    "fallback_us": round(tot(key_passes[0], ("cocluster_assign_kernel",)), 2),
+                                    "fallback_us": round(tot(key_passes[0], ("cocluster_assign_list_kernel",)), 2),
                                     "note": "first iteration: fp16 certified pass + hi/lo fallback; algorithmic "
                                             "FLOP of the reduced form"}
         cand = [pz for pz in key_passes[1:] if "cocluster_score_kernel" in pz["k"]]
@@ -460,7 +460,7 @@ def kernel_table(step, cfg, h, nv, d, qcn, kcn, iters):
                 "lists_us": part(cand, ("cocluster_lists_kernel",)),
                 "score_first_us": part(first, ("cocluster_score_kernel",)),
                 "score_later_us": part(later, ("cocluster_score_kernel",)),
-                "fallback_us": part(cand, ("cocluster_assign_kernel",)),
+                "fallback_us": part(cand, ("cocluster_assign_list_kernel",)),
                 "note": "iterations 2+: triangle-inequality candidates in profile space, exact (same labels)"}
         if full_later:
             stage["key_full_passes_later_avg_us"] = round(
