@@ -391,7 +391,7 @@ __global__ void __launch_bounds__(256) cocluster_prep_mfma_kernel(const uint16_t
     *(uint2*)(lb + (size_t)row * 128 + dd) = make_uint2(lo[0] | ((uint32_t)lo[1] << 16), lo[2] | ((uint32_t)lo[3] << 16));
   };
   if (!e16) {
-    // hi and lo alone: by the lower lanes (shared by both, the 16 columns take 0.5 us longer in a launch of 7 to 14)
+    // hi and lo alone: by the lower lanes (shared with the upper ones a launch of 6 to 14 us takes 0.5 us longer)
     if (!upper && row < jpad) {
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4) {
@@ -508,7 +508,7 @@ __global__ void __launch_bounds__(256) cocluster_prep_mfma_kernel(const uint16_t
 // then a tile-level compare (ties resolve to the lowest cluster index; scores within 2^-19 of each
 // other, below the rounding of the hi + lo sums, are ordered by slot, and for negative scores the
 // higher slot of a tile wins such a near-tie).
-constexpr int kAsgTokWave = 128;
+constexpr int kAsgTokWave = 128;  // tokens of a wave with four column blocks, of a block of waves with one each
 constexpr int kAsgTok = 4 * kAsgTokWave;
 
 // Tokens [t0, t0 + 128 NCB) of a head: of all n tokens, or with LIST entries of the head's token list lst (ntok entries).
